@@ -101,6 +101,10 @@ int lm_launch_app_slots(int S, int64_t N, const uint64_t *bitmap, const uint32_t
 int lm_launch_march(const lm_model *m, const float *rays, const uint64_t *bitmap, const uint32_t *p_first,
                     const uint64_t *word_mask, const uint32_t *ray_list, const uint32_t *bins, uint32_t n_rays, uint32_t *queue, float *w_valid, float *acc,
                     float *depth, uint32_t *app_cnt, uint32_t *p_end, uint32_t *n_marched, hipStream_t st);
+bool lm_rays_kernel_takes(const lm_model *m, int64_t N);
+int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t row, uint32_t cap_valid, uint32_t *app_first,
+                   uint32_t *app_cnt, uint32_t *app_idx, float *app_w, uint32_t cap_app, float *acc, float *depth,
+                   uint32_t *counters, hipStream_t st);
 int lm_launch_basis(int prec, const void *packed, int K, const float *products, uint64_t M, const uint32_t *count,
                     uint32_t cap, float *feat, hipStream_t st);
 
@@ -269,22 +273,31 @@ int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *w
     const uint32_t row = m->ray_row % 8 == 0 ? (uint32_t)m->ray_row : 0u;  // tiles of 8 x 8 pixels need whole tiles per row
     mark(0);
     if (int rc = lm_launch_zero_counters(cnt, st)) return rc;
-    if (int rc = lm_launch_cull_setup(&m->geom, rays, N, w.bitmap, w.p_first, w.ray_list, cnt + LM_STAT_BINS,
-                                      cnt + LM_STAT_N_VALID, w.acc, depth_map, w.app_cnt, w.p_end, row, (uint32_t)w.cap_valid,
-                                      cnt + LM_STAT_OVERFLOW, w.word_mask, st))
-        return rc;
-    mark(LM_STAGE_CULL);
-    // the cull writes word masks for rays of three bitmap words and more (other sample counts take the kernel
-    // with one lane per word, whose rays have one or two words)
-    const uint64_t *masks = (S == 64 || S == 128) ? nullptr : w.word_mask;
-    if (int rc = lm_launch_march(m, rays, w.bitmap, w.p_first, masks, w.ray_list, cnt + LM_STAT_BINS, (uint32_t)N, cnt + LM_STAT_QUEUE,
-                                 w.w_valid, w.acc, depth_map, w.app_cnt, w.p_end, cnt + LM_STAT_N_MARCHED, st))
-        return rc;
-    mark(LM_STAGE_DENSITY);
-    if (int rc = lm_launch_app_slots(S, N, w.bitmap, w.p_first, masks, w.w_valid, m->weight_thres, w.app_cnt, w.p_end,
-                                     w.app_first, w.app_idx, w.app_w, cnt + LM_STAT_N_APP, row, (uint32_t)w.cap_app,
-                                     cnt + LM_STAT_OVERFLOW, st))
-        return rc;
+    if (lm_rays_kernel_takes(m, N)) {
+        // few rays: one kernel up to the appearance list
+        if (int rc = lm_launch_rays(m, rays, (uint32_t)N, row, (uint32_t)w.cap_valid, w.app_first, w.app_cnt, w.app_idx, w.app_w,
+                                    (uint32_t)w.cap_app, w.acc, depth_map, cnt, st))
+            return rc;
+        mark(LM_STAGE_CULL);
+        mark(LM_STAGE_DENSITY);
+    } else {
+        if (int rc = lm_launch_cull_setup(&m->geom, rays, N, w.bitmap, w.p_first, w.ray_list, cnt + LM_STAT_BINS,
+                                          cnt + LM_STAT_N_VALID, w.acc, depth_map, w.app_cnt, w.p_end, row, (uint32_t)w.cap_valid,
+                                          cnt + LM_STAT_OVERFLOW, w.word_mask, st))
+            return rc;
+        mark(LM_STAGE_CULL);
+        // the cull writes word masks for rays of three bitmap words and more (other sample counts take the kernel
+        // with one lane per word, whose rays have one or two words)
+        const uint64_t *masks = (S == 64 || S == 128) ? nullptr : w.word_mask;
+        if (int rc = lm_launch_march(m, rays, w.bitmap, w.p_first, masks, w.ray_list, cnt + LM_STAT_BINS, (uint32_t)N, cnt + LM_STAT_QUEUE,
+                                     w.w_valid, w.acc, depth_map, w.app_cnt, w.p_end, cnt + LM_STAT_N_MARCHED, st))
+            return rc;
+        mark(LM_STAGE_DENSITY);
+        if (int rc = lm_launch_app_slots(S, N, w.bitmap, w.p_first, masks, w.w_valid, m->weight_thres, w.app_cnt, w.p_end,
+                                         w.app_first, w.app_idx, w.app_w, cnt + LM_STAT_N_APP, row, (uint32_t)w.cap_app,
+                                         cnt + LM_STAT_OVERFLOW, st))
+            return rc;
+    }
     mark(LM_STAGE_WEIGHTS);
     if (fused) {
         if (int rc = lm_launch_app_features(m, rays, w.app_idx, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.feat, st)) return rc;

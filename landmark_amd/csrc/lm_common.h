@@ -71,6 +71,12 @@ __device__ __forceinline__ float lm_ray_param(const lm_geom &g, const float *ray
     return tmin;
 }
 
+__device__ __forceinline__ void lm_load_ray(const float *__restrict__ rays, uint64_t r, float *ray) {
+    const float2 *rp2 = reinterpret_cast<const float2 *>(rays + 6 * (size_t)r);
+    const float2 a = rp2[0], b = rp2[1], c = rp2[2];
+    ray[0] = a.x; ray[1] = a.y; ray[2] = b.x; ray[3] = b.y; ray[4] = c.x; ray[5] = c.y;
+}
+
 __device__ __forceinline__ float lm_sample_z(const lm_geom &g, float ray_param, int s) {
     if (g.sampler == LM_SAMPLER_HULL) {
         float b = ray_param * g.tab_t[s];
@@ -200,8 +206,9 @@ __device__ __forceinline__ float lm_alpha_lookup(const lm_geom &g, const float *
 // product of three weights in [0, 1] (never small enough to underflow: a weight is a difference
 // of numbers below 2^24 with spacing >= 2^-24 of their size), so the sum is positive exactly when a
 // set corner has three non-zero weights.  The lower weight (f + 1) - i is never zero; the upper
-// weight i - f is zero when the coordinate is an integer.
-__device__ __forceinline__ bool lm_cells_positive(const lm_geom &g, const float *pt) {
+// weight i - f is zero when the coordinate is an integer.  lm_cells_find gives the cell and the corners that weigh
+// anything (0: the point is outside the table, cell 0), for callers that want several lookups in flight.
+__device__ __forceinline__ size_t lm_cells_find(const lm_geom &g, const float *pt, unsigned &live) {
     float c[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -214,7 +221,7 @@ __device__ __forceinline__ bool lm_cells_positive(const lm_geom &g, const float 
     const float iy = ((c[1] + 1.0f) / 2.0f) * (float)(H - 1);
     const float iz = ((c[2] + 1.0f) / 2.0f) * (float)(D - 1);
     float fx = floorf(ix), fy = floorf(iy), fz = floorf(iz);
-    unsigned live = 0xFFu;
+    live = 0xFFu;
     if (ix - fx == 0.0f) live &= 0x55u;  // corners with xx = 1 weigh nothing
     if (iy - fy == 0.0f) live &= 0x33u;
     if (iz - fz == 0.0f) live &= 0x0Fu;
@@ -222,9 +229,16 @@ __device__ __forceinline__ bool lm_cells_positive(const lm_geom &g, const float 
     fy = fminf(fmaxf(fy, -2.0f), (float)H);
     fz = fminf(fmaxf(fz, -2.0f), (float)D);
     const int x0 = (int)fx, y0 = (int)fy, z0 = (int)fz;
-    if (x0 < -1 || x0 >= W || y0 < -1 || y0 >= H || z0 < -1 || z0 >= D) return false;
-    const size_t ci = ((size_t)(z0 + 1) * (H + 1) + (y0 + 1)) * (W + 1) + (x0 + 1);
-    return (reinterpret_cast<const uint8_t *>(g.vol)[ci] & live) != 0u;
+    if (x0 < -1 || x0 >= W || y0 < -1 || y0 >= H || z0 < -1 || z0 >= D) {
+        live = 0u;
+        return 0;
+    }
+    return ((size_t)(z0 + 1) * (H + 1) + (y0 + 1)) * (W + 1) + (x0 + 1);
+}
+__device__ __forceinline__ bool lm_cells_positive(const lm_geom &g, const float *pt) {
+    unsigned live;
+    const size_t ci = lm_cells_find(g, pt, live);
+    return live != 0u && (reinterpret_cast<const uint8_t *>(g.vol)[ci] & live) != 0u;
 }
 
 // Sample validity = inside the AABB and (no volume or lookup > threshold)
@@ -248,6 +262,13 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
 __device__ __forceinline__ unsigned lm_lane() { return __lane_id(); }
 __device__ __forceinline__ unsigned lm_mbcnt(uint64_t mask) {  // set bits of mask below this lane
     return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
+// Orders a wave's LDS accesses before and after this point (they complete in order; the fences only pin the compiler)
+__device__ __forceinline__ void lm_wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Rays waiting for the marching kernel are kept in four lists by their number of valid samples
