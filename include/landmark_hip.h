@@ -278,6 +278,13 @@ int lm_mlp_pack_bias1(const float *b1, float *packed_b1_out);
 /* feat [M,27] fp32, view [M,3] fp32 -> rgb [M,3] fp32 */
 int lm_mlp(int32_t prec, const void *packed, int32_t K_basis, const float *feat, const float *view, int64_t M,
            float *rgb, void *stream);
+/* compute_appfeature in one kernel: normalised points xyz [M,3] -> feat [M,27] = basis_mat(plane * line products),
+ * gridnerf_sequential.py:829-871, with the basis_mat of `packed` (mode `prec`).  Covers planes of equal channel count
+ * (16, 32, 48 or 64) whose basis_mat fits LDS: lm_app_features_xyz_supported() returns 1.  Other models take
+ * lm_gather_app_xyz + lm_basis, which give the same features. */
+int lm_app_features_xyz_supported(const lm_plane *planes, int32_t n_planes, int32_t prec);
+int lm_app_features_xyz(const lm_plane *planes, int32_t n_planes, int32_t prec, const void *packed, const float *xyz,
+                        int64_t M, float *feat, void *stream);
 /* products [M,K] fp32 -> feat [M,27] fp32 : basis_mat(products), gridnerf_sequential.py:871 */
 int lm_basis(int32_t prec, const void *packed, int32_t K_basis, const float *products, int64_t M, float *feat,
              void *stream);

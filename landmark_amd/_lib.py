@@ -74,6 +74,8 @@ SYMBOLS = {
     "lm_mlp_bias1_offset": (_SZ, [_I32, _I32]),
     "lm_mlp_pack_bias1": (C.c_int, [_P, _P]),
     "lm_mlp": (C.c_int, [_I32, _P, _I32, _P, _P, _I64, _P, _P]),
+    "lm_app_features_xyz_supported": (C.c_int, [C.POINTER(LmPlane), _I32, _I32]),
+    "lm_app_features_xyz": (C.c_int, [C.POINTER(LmPlane), _I32, _I32, _P, _P, _I64, _P, _P]),
     "lm_basis": (C.c_int, [_I32, _P, _I32, _P, _I64, _P, _P]),
     "lm_weights": (C.c_int, [C.POINTER(LmGeom), _P, _I64, _P, _P, _P, _F, _F, _F, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "lm_composite_rgb": (C.c_int, [_I64, _P, _P, _P, _P, _P, _I32, _P, _P]),

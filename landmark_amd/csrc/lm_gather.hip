@@ -290,10 +290,13 @@ template <int PREC> struct AppFeatBlock { static constexpr int N = 512; };
 // LDS: [basis fragments | one product tile per wave].  A tile is 32 samples x (C + 4) floats.
 __host__ __device__ inline size_t app_feat_tile_bytes(int C) { return (size_t)32 * (C + 4) * sizeof(float); }
 
-template <int PREC, typename T, int NU>  // NU = groups of 16 channels per plane (C = 16 * NU)
+// XYZ: the samples are M_host points given by their normalised coordinates (`rays` = xyz[M][3]) instead of list entries.
+// Products through memory and a second kernel for basis_mat instead (k_app_xyz + k_basis) take 2.60 ms for 2^20 random
+// points of nine 48-channel planes, 1.8 GB of products written and read again; this kernel takes 1.41 ms.
+template <int PREC, typename T, int NU, bool XYZ>  // NU = groups of 16 channels per plane (C = 16 * NU)
 __global__ __launch_bounds__(AppFeatBlock<PREC>::N) void k_app_feat(lm_geom g, PlaneSet ps, int K,
                                                                    const char *__restrict__ packed, lm_mma::PackLayout L,
-                                                                   const float *__restrict__ rays,
+                                                                   const float *__restrict__ rays, uint64_t M_host,
                                                                    const uint32_t *__restrict__ list,
                                                                    const uint32_t *__restrict__ count, uint32_t cap,
                                                                    float *__restrict__ feat) {
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(AppFeatBlock<PREC>::N) void k_app_feat(lm_geom g, P
     const unsigned lane = lm_lane(), j = lane & 31u, h = lane >> 5;
     const unsigned qlane = lane & 3u, gs = lane >> 2;  // gather role: 4 lanes per sample, 16 samples per pass
     float *tile = reinterpret_cast<float *>(lds + basis_bytes + (threadIdx.x / LM_WAVE) * app_feat_tile_bytes(C));
-    const uint64_t M = min(*count, cap);  // the counter keeps counting past the list's capacity
+    const uint64_t M = XYZ ? M_host : (uint64_t)min(*count, cap);  // the counter keeps counting past the list's capacity
     const uint64_t n_tiles = (M + 31) / 32;
     constexpr unsigned kWaves = AppFeatBlock<PREC>::N / LM_WAVE;
     const uint64_t wave_id = (uint64_t)lm_xcd_swizzle(blockIdx.x, gridDim.x) * kWaves + threadIdx.x / LM_WAVE;
@@ -326,9 +329,15 @@ __global__ __launch_bounds__(AppFeatBlock<PREC>::N) void k_app_feat(lm_geom g, P
         // the two samples this lane gathers for (pass 0: tile row gs, pass 1: row 16 + gs)
         float q0[4], q1[4];
         {
-            const uint64_t p0 = tile_id * 32 + gs, p1 = p0 + 16;
-            list_coords(g, rays, list[p0 < M ? p0 : M - 1], q0);
-            list_coords(g, rays, list[p1 < M ? p1 : M - 1], q1);
+            const uint64_t p0 = tile_id * 32 + gs, p1 = p0 + 16, c0 = p0 < M ? p0 : M - 1, c1 = p1 < M ? p1 : M - 1;
+            if constexpr (XYZ) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) { q0[i] = rays[3 * c0 + i]; q1[i] = rays[3 * c1 + i]; }
+                q0[3] = q1[3] = 0.0f;
+            } else {
+                list_coords(g, rays, list[c0], q0);
+                list_coords(g, rays, list[c1], q1);
+            }
         }
         floatx16 acc;
 #pragma unroll
@@ -435,20 +444,26 @@ __global__ __launch_bounds__(AppFeatBlock<PREC>::N) void k_app_feat(lm_geom g, P
     }
 }
 
-template <int PREC, typename T>
-int launch_app_feat(int nu, const lm_model *m, const PlaneSet &ps, int K, const float *rays, const uint32_t *list,
-                    const uint32_t *count, uint32_t cap, float *feat, hipStream_t st) {
+size_t app_feat_lds(int prec, int K, int C) {
+    using namespace lm_mma;
+    const size_t elem = prec == LM_MLP_F32 || prec == LM_MLP_F16X2 ? 4 : 2;  // F16X2: two parts
+    return (size_t)32 * K * elem + (AppFeatBlock<LM_MLP_F16>::N / LM_WAVE) * app_feat_tile_bytes(C);
+}
+
+template <int PREC, typename T, bool XYZ>
+int launch_app_feat(int nu, const lm_geom &geom, const void *packed, const PlaneSet &ps, int K, const float *rays, uint64_t M,
+                    const uint32_t *list, const uint32_t *count, uint32_t cap, float *feat, hipStream_t st) {
     using namespace lm_mma;
     const PackLayout L = pack_layout(PREC, K);
     constexpr int kThreads = AppFeatBlock<PREC>::N;
-    const size_t basis = (size_t)32 * K * sizeof(typename Mma<PREC>::elem) * Mma<PREC>::NP;
-    const size_t lds = basis + (kThreads / LM_WAVE) * app_feat_tile_bytes(16 * nu);
+    const size_t lds = app_feat_lds(PREC, K, 16 * nu);
     if (lds > 160 * 1024) LM_FAIL(LM_ERR_UNSUPPORTED, "basis_mat fragments + tiles (%zu bytes) do not fit LDS", lds);
     const unsigned per_cu = (unsigned)std::max<size_t>(1, std::min<size_t>(2, (size_t)(160 * 1024) / lds));
-    const unsigned grid = (unsigned)lm_persistent_blocks((int)per_cu);
+    unsigned grid = (unsigned)lm_persistent_blocks((int)per_cu);
+    if (XYZ) grid = (unsigned)std::min<uint64_t>(grid, (M + 31) / 32);  // few points: a tile per workgroup
 #define LM_AF_CASE(NU_)                                                                                            \
     case NU_: {                                                                                                    \
-        auto kern = &k_app_feat<PREC, T, NU_>;                                                                     \
+        auto kern = &k_app_feat<PREC, T, NU_, XYZ>;                                                                \
         static thread_local size_t reserved_on[LM_MAX_DEVICES] = {}; /* set once per thread, device, kernel, size */ \
         size_t &reserved = reserved_on[lm_current_device()];                                                       \
         if (reserved != lds) {                                                                                     \
@@ -458,7 +473,7 @@ int launch_app_feat(int nu, const lm_model *m, const PlaneSet &ps, int K, const 
                 LM_FAIL(LM_ERR_LAUNCH, "k_app_feat: LDS reservation failed: %s", hipGetErrorString(e));            \
             reserved = lds;                                                                                        \
         }                                                                                                          \
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, st, m->geom, ps, K, (const char *)m->mlp_packed, L, rays, \
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, st, geom, ps, K, (const char *)packed, L, rays, M, \
                            list, count, cap, feat);                                                                \
         break;                                                                                                     \
     }
@@ -625,13 +640,14 @@ extern "C" int lm_app_products(const lm_model *m, const float *rays, const uint3
     return lm_launch_app_products(m, rays, app_idx, counters + LM_STAT_N_APP, UINT32_MAX, products, (hipStream_t)stream);
 }
 
-// True when the fused gather + basis_mat kernel covers this model's appearance planes.
-int lm_app_feat_supported(const lm_model *m) {
-    const int C = m->app[0].C;
-    for (int k = 0; k < m->n_planes; ++k)
-        if (m->app[k].C != C) return 0;
+// True when the fused gather + basis_mat kernel covers these appearance planes.
+static int app_feat_covers(const lm_plane *planes, int n) {
+    const int C = planes[0].C;
+    for (int k = 0; k < n; ++k)
+        if (planes[k].C != C) return 0;
     return C % 16 == 0 && C >= 16 && C <= 64;
 }
+int lm_app_feat_supported(const lm_model *m) { return app_feat_covers(m->app, m->n_planes); }
 
 int lm_check_prec(int prec);
 int lm_check_K(int K);
@@ -643,6 +659,26 @@ extern "C" int lm_app_features(const lm_model *m, const float *rays, const uint3
                                float *feat, void *stream) {
     LM_REQUIRE(counters != nullptr, "counters is null");
     return lm_launch_app_features(m, rays, app_idx, counters + LM_STAT_N_APP, UINT32_MAX, feat, (hipStream_t)stream);
+}
+
+template <bool XYZ>
+static int app_features(int prec, int dtype, int nu, const lm_geom &geom, const void *packed, const PlaneSet &ps, int K,
+                        const float *rays, uint64_t M, const uint32_t *app_idx, const uint32_t *cnt, uint32_t cap, float *feat,
+                        hipStream_t st) {
+#define LM_AF_ONE(PREC_, T_) launch_app_feat<PREC_, T_, XYZ>(nu, geom, packed, ps, K, rays, M, app_idx, cnt, cap, feat, st)
+#define LM_AF_GO(PREC_)                                                                                         \
+    return dtype == LM_F32 ? LM_AF_ONE(PREC_, float)                                                            \
+           : nu == 3       ? LM_AF_ONE(PREC_, Half6)                                                            \
+           : (nu & 1)      ? LM_AF_ONE(PREC_, Half4)                                                            \
+                           : LM_AF_ONE(PREC_, __half)
+    switch (prec) {
+        case LM_MLP_F32: LM_AF_GO(LM_MLP_F32);
+        case LM_MLP_F16: LM_AF_GO(LM_MLP_F16);
+        case LM_MLP_BF16: LM_AF_GO(LM_MLP_BF16);
+        default: LM_AF_GO(LM_MLP_F16X2);
+    }
+#undef LM_AF_GO
+#undef LM_AF_ONE
 }
 
 int lm_launch_app_features(const lm_model *m, const float *rays, const uint32_t *app_idx, const uint32_t *cnt, uint32_t cap,
@@ -658,19 +694,29 @@ int lm_launch_app_features(const lm_model *m, const float *rays, const uint32_t 
     if (!lm_app_feat_supported(m))
         LM_FAIL(LM_ERR_UNSUPPORTED, "fused appearance gather needs equal channel counts of 16..64 in steps of 16");
     const PlaneSet ps = make_set(m->app, m->n_planes, &m->geom);
-    const int nu = m->app[0].C / 16;
-#define LM_AF_GO(PREC_)                                                                                         \
-    return dtype == LM_F32 ? launch_app_feat<PREC_, float>(nu, m, ps, K, rays, app_idx, cnt, cap, feat, st)     \
-           : nu == 3       ? launch_app_feat<PREC_, Half6>(nu, m, ps, K, rays, app_idx, cnt, cap, feat, st)     \
-           : (nu & 1)      ? launch_app_feat<PREC_, Half4>(nu, m, ps, K, rays, app_idx, cnt, cap, feat, st)     \
-                           : launch_app_feat<PREC_, __half>(nu, m, ps, K, rays, app_idx, cnt, cap, feat, st)
-    switch (m->mlp_prec) {
-        case LM_MLP_F32: LM_AF_GO(LM_MLP_F32);
-        case LM_MLP_F16: LM_AF_GO(LM_MLP_F16);
-        case LM_MLP_BF16: LM_AF_GO(LM_MLP_BF16);
-        default: LM_AF_GO(LM_MLP_F16X2);
-    }
-#undef LM_AF_GO
+    return app_features<false>(m->mlp_prec, dtype, m->app[0].C / 16, m->geom, m->mlp_packed, ps, K, rays, 0, app_idx, cnt, cap,
+                               feat, st);
+}
+
+extern "C" int lm_app_features_xyz_supported(const lm_plane *planes, int32_t n_planes, int32_t prec) {
+    int dtype, K;
+    if (lm_check_planes(planes, n_planes, &dtype, &K) || lm_check_prec(prec) || lm_check_K(K)) return 0;
+    return app_feat_covers(planes, n_planes) && app_feat_lds(prec, K, planes[0].C) <= 160 * 1024;
+}
+
+extern "C" int lm_app_features_xyz(const lm_plane *planes, int32_t n_planes, int32_t prec, const void *packed, const float *xyz,
+                                   int64_t M, float *feat, void *stream) {
+    int dtype, K;
+    if (int rc = lm_check_planes(planes, n_planes, &dtype, &K)) return rc;
+    if (int rc = lm_check_prec(prec)) return rc;
+    if (int rc = lm_check_K(K)) return rc;
+    LM_REQUIRE(M >= 0, "negative count");
+    if (M == 0) return LM_OK;
+    LM_REQUIRE(packed && xyz && feat && lm_aligned16(packed), "null or misaligned buffer");
+    if (!lm_app_features_xyz_supported(planes, n_planes, prec))
+        LM_FAIL(LM_ERR_UNSUPPORTED, "needs equal channel counts of 16..64 in steps of 16 and a basis_mat that fits LDS (K %d)", K);
+    return app_features<true>(prec, dtype, planes[0].C / 16, lm_geom{}, packed, make_set(planes, n_planes), K, xyz, (uint64_t)M,
+                              nullptr, nullptr, 0u, feat, (hipStream_t)stream);
 }
 
 // Density + transmittance march over the rays listed in ray_list (those with valid samples).

@@ -749,7 +749,15 @@ class GridNeRFHIP:
     @torch.no_grad()
     def compute_appfeature(self, xyz_sampled, precision=None):
         """GridNeRF.compute_appfeature: basis_mat(products) -> [M,27]."""
-        return self.basis(self.app_products(xyz_sampled), precision)
+        prec, packed = self._pack_mlp(precision or self.mlp_precision)
+        arr = self._plane_array(self._app)
+        if not self.lib.lm_app_features_xyz_supported(arr, len(self._app), prec):
+            return self.basis(self.app_products(xyz_sampled), precision)
+        xyz = xyz_sampled.to(self.device, torch.float32).contiguous()
+        M = xyz.shape[0]
+        out = torch.empty((M, 27), dtype=torch.float32, device=self.device)
+        L.check(self.lib.lm_app_features_xyz(arr, len(self._app), prec, packed.data_ptr(), xyz.data_ptr(), M, out.data_ptr(), L.current_stream()), "lm_app_features_xyz")
+        return out
 
     @torch.no_grad()
     def render_module(self, viewdirs, features, precision=None, app_code=None):
