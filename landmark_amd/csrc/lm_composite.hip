@@ -9,7 +9,7 @@
 // counts those above the threshold, a wave-wide prefix sum plus one atomic per wave reserves
 // a contiguous slot range per ray in the appearance list, the second pass fills the slots.
 // A ray's slots are therefore contiguous and in sample order.
-// k_composite: one lane per ray sums weight * rgb over its slots, adds the white
+// k_composite: a quad per ray sums weight * rgb over its slots, adds the white
 // background and clamps.
 // In the whole-chunk render the weights come from the marching kernel (density gather fused with
 // the transmittance walk); k_app_slots then builds the appearance list from the stored weights the
@@ -26,11 +26,8 @@ constexpr int kBlock = 256;
 #ifndef LM_SLOTS_STAGE
 #define LM_SLOTS_STAGE 4096
 #endif
-#ifndef LM_COMPOSITE_STAGE
-#define LM_COMPOSITE_STAGE 512
-#endif
-// list entries a wave moves through LDS: k_app_slots its whole range at once, k_composite a window at a time
-constexpr int kSlotsStage = LM_SLOTS_STAGE, kCompositeStage = LM_COMPOSITE_STAGE;
+// list entries a wave of k_app_slots moves through LDS at once
+constexpr int kSlotsStage = LM_SLOTS_STAGE;
 
 __global__ __launch_bounds__(kBlock) void k_weights(lm_geom g, const float *__restrict__ rays, uint64_t N,
                                                     const uint64_t *__restrict__ bitmap,
@@ -113,117 +110,47 @@ __global__ __launch_bounds__(kBlock) void k_weights(lm_geom g, const float *__re
     }
 }
 
-// The appearance list is laid out wave by wave: the 64 rays a wave handles (consecutive positions of the visiting
-// order) own one contiguous range of slots.  k_app_slots and k_composite are one lane per ray, so a lane's slots
-// are a short run somewhere in that range: written or read directly, every access of the wave touches 64 different
-// cache lines, each of which is visited again a few entries later (partial-line writes reach the memory several
-// times over).  Both kernels therefore move the wave's range through LDS (k_app_slots when it has at most STAGE
-// entries, k_composite in windows of STAGE): the lanes work on the LDS copy in their own order, the wave copies
-// the range to or from memory in whole lines.  A workgroup is one wave.
-template <int STAGE>
-__global__ __launch_bounds__(LM_WAVE) void k_composite(uint64_t N, const uint32_t *__restrict__ app_first,
-                                                       const uint32_t *__restrict__ app_cnt,
-                                                       const float *__restrict__ app_w, const float *__restrict__ rgb,
-                                                       const float *__restrict__ acc, int white_bg, uint32_t row,
-                                                       float *__restrict__ rgb_map) {
-    __shared__ float s_w[STAGE];
-    __shared__ float s_c[3 * STAGE];
-    const unsigned lane = lm_lane();
-    const uint64_t o = (uint64_t)blockIdx.x * LM_WAVE + lane;
-    const bool live = o < N;
-    const uint64_t r = live ? lm_ray_order((uint32_t)o, (uint32_t)N, row) : 0;
-    const uint32_t first = live ? app_first[r] : 0u, n = live ? app_cnt[r] : 0u;
-    // the slots this wave reads: [lo, hi) over its rays that have any
-    uint32_t lo = n ? first : 0xFFFFFFFFu, hi = n ? first + n : 0u;
+// A quad per ray, a lane per colour channel: a quad's loads fall into one run of the list whatever the order the rays'
+// ranges lie in, sixteen entries in flight.  A lane per ray, with the wave's range of the list staged through LDS in
+// windows, waits for each window and does badly where neighbouring rays' ranges lie apart (k_rays reserves four rays at a
+// time): 8192 rays of 30 entries 13 - 75 -> 5.8 us, 4096 rays of 5 entries 13 -> 5 us, 518400 rays of 57 entries 390 -> 223 us,
+// a million rays of 11 entries 74 us either way.  Eight entries in flight: 7.1, 5.1, 279, 81 us.
+__global__ __launch_bounds__(kBlock) void k_composite(uint64_t N, const uint32_t *__restrict__ app_first,
+                                                           const uint32_t *__restrict__ app_cnt, const float *__restrict__ app_w,
+                                                           const float *__restrict__ rgb, const float *__restrict__ acc, int white_bg,
+                                                           uint32_t row, float *__restrict__ rgb_map) {
+    const uint64_t o = (uint64_t)blockIdx.x * (kBlock / 4) + threadIdx.x / 4;
+    const unsigned ch = threadIdx.x & 3u;
+    if (o >= N || ch == 3u) return;
+    const uint64_t r = lm_ray_order((uint32_t)o, (uint32_t)N, row);
+    constexpr uint32_t kAhead = 16;
+    const uint32_t n = app_cnt[r];
+    const size_t first = app_first[r];
+    const float a = white_bg ? acc[r] : 0.0f;
+    const float *w = app_w + first, *c = rgb + 3 * first + ch;
+    float sum = 0.0f;
+    for (uint32_t i = 0; i < n; i += kAhead) {
+        float wv[kAhead], cv[kAhead];
 #pragma unroll
-    for (int d = 1; d < LM_WAVE; d <<= 1) {
-        lo = min(lo, (uint32_t)__shfl_xor((int)lo, d));
-        hi = max(hi, (uint32_t)__shfl_xor((int)hi, d));
-    }
-    // Windows of STAGE slots over [lo, hi): the wave loads a window in whole lines, every lane adds its slots of
-    // that window.  Windows ascend, so a lane's sum keeps the slot order.  A layout whose ranges lie far apart
-    // (hi - lo much larger than the slots in use) is read directly instead.
-    uint32_t used = n;
-#pragma unroll
-    for (int d = 1; d < LM_WAVE; d <<= 1) used += (uint32_t)__shfl_xor((int)used, d);
-    const bool staged = hi > lo && (uint64_t)(hi - lo) <= 2ull * used + STAGE;
-    float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
-    if (staged) {
-        for (uint64_t win = lo; win < hi; win += STAGE) {  // 64-bit: hi may be within STAGE of 2^32
-            const uint32_t len = (uint32_t)min((uint64_t)STAGE, hi - win);
-            if (win != lo) __builtin_amdgcn_wave_barrier();  // every lane is done with the previous window
-            // four loads in flight per lane and array (indices past the window repeat its last entry)
-            constexpr int kAhead = 4;
-            for (uint32_t i0 = 0; i0 < 3u * len; i0 += kAhead * LM_WAVE) {
-                float c[kAhead], w[kAhead];
-#pragma unroll
-                for (int u = 0; u < kAhead; ++u) {
-                    const uint32_t i = i0 + u * LM_WAVE + lane;
-                    c[u] = rgb[3 * (size_t)win + min(i, 3u * len - 1u)];
-                    if (i0 < len) w[u] = app_w[win + min(i, len - 1u)];
-                }
-#pragma unroll
-                for (int u = 0; u < kAhead; ++u) {
-                    const uint32_t i = i0 + u * LM_WAVE + lane;
-                    if (i < 3u * len) s_c[i] = c[u];
-                    if (i < len) s_w[i] = w[u];
-                }
-            }
-            // LDS operations of one wave complete in order; the fences only pin the compiler
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (n) {
-                const uint64_t from = max((uint64_t)first, win), to = min((uint64_t)first + n, win + len);
-                // four entries per trip, their LDS reads issued together; the sums stay in slot order
-                constexpr int kTrip = 4;
-                for (uint64_t q = from; q < to; q += kTrip) {
-                    float w[kTrip], c[kTrip][3];
-#pragma unroll
-                    for (int u = 0; u < kTrip; ++u) {
-                        const uint32_t at = (uint32_t)(min(q + u, to - 1) - win);
-                        w[u] = s_w[at];
-                        c[u][0] = s_c[3 * at]; c[u][1] = s_c[3 * at + 1]; c[u][2] = s_c[3 * at + 2];
-                    }
-#pragma unroll
-                    for (int u = 0; u < kTrip; ++u)
-                        if (q + u < to) {
-                            c0 = fmaf(w[u], c[u][0], c0); c1 = fmaf(w[u], c[u][1], c1); c2 = fmaf(w[u], c[u][2], c2);
-                        }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            const uint32_t at = min(i + u, n - 1u);
+            wv[u] = w[at];
+            cv[u] = c[3 * (size_t)at];
         }
-    } else if (live) {
-        // eight slots per trip, all loads issued before the sums (which stay in slot order)
-        constexpr int kBatch = 8;
-        for (uint32_t i = 0; i < n; i += kBatch) {
-            float w[kBatch], c[kBatch][3];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t s = first + (i + u < n ? i + u : n - 1);
-                w[u] = app_w[s];
-                c[u][0] = rgb[3 * (size_t)s]; c[u][1] = rgb[3 * (size_t)s + 1]; c[u][2] = rgb[3 * (size_t)s + 2];
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                if (i + u < n) {
-                    c0 = fmaf(w[u], c[u][0], c0); c1 = fmaf(w[u], c[u][1], c1); c2 = fmaf(w[u], c[u][2], c2);
-                }
-        }
+        for (uint32_t u = 0; u < kAhead; ++u)
+            if (i + u < n) sum = fmaf(wv[u], cv[u], sum);
     }
-    if (!live) return;
-    if (white_bg) {
-        const float bgd = 1.0f - acc[r];
-        c0 += bgd; c1 += bgd; c2 += bgd;
-    }
-    rgb_map[3 * r + 0] = fminf(fmaxf(c0, 0.0f), 1.0f);
-    rgb_map[3 * r + 1] = fminf(fmaxf(c1, 0.0f), 1.0f);
-    rgb_map[3 * r + 2] = fminf(fmaxf(c2, 0.0f), 1.0f);
+    if (white_bg) sum += 1.0f - a;
+    rgb_map[3 * r + ch] = fminf(fmaxf(sum, 0.0f), 1.0f);
 }
 
 // Appearance list from stored weights: a contiguous slot range per ray (wave prefix + one
 // atomic), filled in sample order from the weights of the ray's samples [first, p_end).
+// The 64 rays a wave handles own one contiguous range of slots, a lane's slots are a short run somewhere in it: written
+// directly, every access of the wave touches 64 different cache lines, each visited again a few entries later
+// (partial-line writes reach the memory several times over).  A range of at most STAGE entries is therefore put together
+// in LDS and written in whole lines.  A workgroup is one wave.
 template <int STAGE>
 __global__ __launch_bounds__(LM_WAVE) void k_app_slots(int S, uint64_t N, const uint64_t *__restrict__ bitmap,
                                                        const uint32_t *__restrict__ p_first,
@@ -335,9 +262,8 @@ int lm_launch_composite(int64_t N, const uint32_t *app_first, const uint32_t *ap
                         const float *rgb, const float *acc, int white_bg, uint32_t row, float *rgb_map,
                         hipStream_t stream) {
     if (N == 0) return LM_OK;
-    const unsigned grid = (unsigned)(((uint64_t)N + LM_WAVE - 1) / LM_WAVE);
-    hipLaunchKernelGGL(k_composite<kCompositeStage>, dim3(grid), dim3(LM_WAVE), 0, stream, (uint64_t)N, app_first, app_cnt, app_w, rgb,
-                       acc, white_bg, row, rgb_map);
+    hipLaunchKernelGGL(k_composite, dim3((unsigned)(((uint64_t)N + kBlock / 4 - 1) / (kBlock / 4))), dim3(kBlock), 0, stream,
+                       (uint64_t)N, app_first, app_cnt, app_w, rgb, acc, white_bg, row, rgb_map);
     LM_CHECK_LAUNCH("k_composite");
     return LM_OK;
 }
