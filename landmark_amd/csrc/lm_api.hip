@@ -105,6 +105,9 @@ bool lm_rays_kernel_takes(const lm_model *m, int64_t N);
 int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t row, uint32_t cap_valid, uint32_t *app_first,
                    uint32_t *app_cnt, uint32_t *app_idx, float *app_w, uint32_t cap_app, float *acc, float *depth,
                    uint32_t *counters, hipStream_t st);
+bool lm_shade_takes(const lm_model *m, int64_t N, int K);
+int lm_launch_shade(const lm_model *m, const float *rays, const uint32_t *list, const uint32_t *count, uint32_t cap, float *rgb,
+                    hipStream_t st);
 int lm_launch_basis(int prec, const void *packed, int K, const float *products, uint64_t M, const uint32_t *count,
                     uint32_t cap, float *feat, hipStream_t st);
 
@@ -273,7 +276,8 @@ int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *w
     const uint32_t row = m->ray_row % 8 == 0 ? (uint32_t)m->ray_row : 0u;  // tiles of 8 x 8 pixels need whole tiles per row
     mark(0);
     if (int rc = lm_launch_zero_counters(cnt, st)) return rc;
-    if (lm_rays_kernel_takes(m, N)) {
+    const bool few = lm_rays_kernel_takes(m, N);
+    if (few) {
         // few rays: one kernel up to the appearance list
         if (int rc = lm_launch_rays(m, rays, (uint32_t)N, row, (uint32_t)w.cap_valid, w.app_first, w.app_cnt, w.app_idx, w.app_w,
                                     (uint32_t)w.cap_app, w.acc, depth_map, cnt, st))
@@ -299,18 +303,24 @@ int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *w
             return rc;
     }
     mark(LM_STAGE_WEIGHTS);
-    if (fused) {
-        if (int rc = lm_launch_app_features(m, rays, w.app_idx, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.feat, st)) return rc;
+    if (few && lm_shade_takes(m, N, K)) {
+        // few samples: gather, basis_mat and colour network in one kernel
+        if (int rc = lm_launch_shade(m, rays, w.app_idx, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.rgb, st)) return rc;
+        mark(LM_STAGE_APP);
     } else {
-        // channel counts the fused kernel does not cover: products through memory, then basis_mat
-        if (int rc = lm_launch_app_products(m, rays, w.app_idx, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.products, st)) return rc;
-        if (int rc = lm_launch_basis(m->mlp_prec, m->mlp_packed, K, w.products, 0, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.feat, st))
+        if (fused) {
+            if (int rc = lm_launch_app_features(m, rays, w.app_idx, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.feat, st)) return rc;
+        } else {
+            // channel counts the fused kernel does not cover: products through memory, then basis_mat
+            if (int rc = lm_launch_app_products(m, rays, w.app_idx, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.products, st)) return rc;
+            if (int rc = lm_launch_basis(m->mlp_prec, m->mlp_packed, K, w.products, 0, cnt + LM_STAT_N_APP, (uint32_t)w.cap_app, w.feat, st))
+                return rc;
+        }
+        mark(LM_STAGE_APP);
+        if (int rc = lm_launch_app_colour(m->mlp_prec, m->mlp_packed, K, S, w.feat, rays, w.app_idx, cnt + LM_STAT_N_APP,
+                                          (uint32_t)w.cap_app, w.rgb, st))
             return rc;
     }
-    mark(LM_STAGE_APP);
-    if (int rc = lm_launch_app_colour(m->mlp_prec, m->mlp_packed, K, S, w.feat, rays, w.app_idx, cnt + LM_STAT_N_APP,
-                                      (uint32_t)w.cap_app, w.rgb, st))
-        return rc;
     mark(LM_STAGE_COLOUR);
     if (int rc = lm_launch_composite(N, w.app_first, w.app_cnt, w.app_w, w.rgb, w.acc, m->white_bg, row, rgb_map, st)) return rc;
     mark(LM_STAGE_COMPOSITE);

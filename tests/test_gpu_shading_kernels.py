@@ -1,6 +1,7 @@
-"""compute_appfeature has two forms: one kernel from points to features, and products through memory with basis_mat after
-them.  Both do the same operations in the same order and agree exactly, in every arithmetic mode and for every channel width
-and storage type the one kernel covers; a basis_mat too large for it takes the other form."""
+"""The back half of a render has two forms: one kernel per stage (large chunks) and one kernel from appearance entries to
+colours (small chunks).  Both do the same operations in the same order, so pictures agree exactly, in every arithmetic mode
+and for every channel width, storage type and number of planes the small form covers; widths and mixtures it does not cover
+take the kernels per stage.  compute_appfeature has the same two forms: one kernel, and products through memory."""
 import pytest
 import torch
 
@@ -16,6 +17,23 @@ def _scene(an, ndims, res=(1,), fp16=False, seed=7):
     for t in p.density_plane:
         t.mul_(6.0)
     return O.to_fp16_features(p) if fp16 else p
+
+
+@pytest.mark.parametrize("net", ["f32", "f16x2", "f16", "bf16"])
+@pytest.mark.parametrize("an,ndims,res,fp16", [(16, 1, (1,), False), (32, 3, (1,), False), (48, 3, (1, 2, 4), False), (64, 3, (1, 2), False),
+                                               (16, 3, (1,), True), (32, 1, (1, 2), True), (48, 3, (1,), True), (64, 3, (1,), True)])
+def test_small_chunk_shading_equals_the_stage_kernels(gpu_lib, net, an, ndims, res, fp16):
+    from landmark_amd.model import GridNeRFHIP
+
+    m = GridNeRFHIP(_scene(an, ndims, res, fp16), device="cuda", mlp_precision=net)
+    rays = scenes.pinhole_rays(120, 110, 100.0, scenes.sphere_pose(2.5, 9)).cuda()  # 13200 rays: kernels per stage
+    whole, _ = m(rays, chunk=rays.shape[0])
+    assert m.last_counts()["n_app"] > 1000 and (whole["rgb_map"] < 0.99).any()
+    at = 6000  # the middle of the picture
+    for n in (1, 2, 31, 500, 4096):  # fewer and more than 32 entries, many tiles per workgroup
+        part, _ = m(rays[at : at + n], chunk=n)
+        assert torch.equal(part["rgb_map"], whole["rgb_map"][at : at + n])
+        assert torch.equal(part["depth_map"], whole["depth_map"][at : at + n])
 
 
 @pytest.mark.parametrize("net", ["f32", "f16x2", "f16", "bf16"])
