@@ -698,6 +698,10 @@ int lm_launch_app_features(const lm_model *m, const float *rays, const uint32_t 
                                feat, st);
 }
 
+bool lm_few_points_take(int prec, int K, int64_t M);
+int lm_launch_few_points(const lm_plane *planes, int n, int prec, int dtype, int K, const void *packed, const float *xyz, uint32_t M,
+                         float *feat, hipStream_t st);
+
 extern "C" int lm_app_features_xyz_supported(const lm_plane *planes, int32_t n_planes, int32_t prec) {
     int dtype, K;
     if (lm_check_planes(planes, n_planes, &dtype, &K) || lm_check_prec(prec) || lm_check_K(K)) return 0;
@@ -715,6 +719,7 @@ extern "C" int lm_app_features_xyz(const lm_plane *planes, int32_t n_planes, int
     LM_REQUIRE(packed && xyz && feat && lm_aligned16(packed), "null or misaligned buffer");
     if (!lm_app_features_xyz_supported(planes, n_planes, prec))
         LM_FAIL(LM_ERR_UNSUPPORTED, "needs equal channel counts of 16..64 in steps of 16 and a basis_mat that fits LDS (K %d)", K);
+    if (lm_few_points_take(prec, K, M)) return lm_launch_few_points(planes, n_planes, prec, dtype, K, packed, xyz, (uint32_t)M, feat, (hipStream_t)stream);
     return app_features<true>(prec, dtype, planes[0].C / 16, lm_geom{}, packed, make_set(planes, n_planes), K, xyz, (uint64_t)M,
                               nullptr, nullptr, 0u, feat, (hipStream_t)stream);
 }

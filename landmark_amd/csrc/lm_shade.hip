@@ -94,10 +94,11 @@ template <int PREC> struct ShadeLds {
     __host__ __device__ static size_t total(int K) { return first(K) + kIn2; }
 };
 
-template <int PREC, typename T, int NU>  // NU = groups of 16 channels per plane
+// FEAT: the first half only, points to features: `rays` = xyz[M_host][3], `rgb` = feat[M_host][27]
+template <int PREC, typename T, int NU, bool FEAT>  // NU = groups of 16 channels per plane
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_shade(
     lm_geom g, PlaneSet ps, int K, const char *__restrict__ packed, PackLayout L, const float *__restrict__ rays,
-    const uint32_t *__restrict__ list, const uint32_t *__restrict__ count, uint32_t cap, float *__restrict__ rgb) {
+    uint32_t M_host, const uint32_t *__restrict__ list, const uint32_t *__restrict__ count, uint32_t cap, float *__restrict__ rgb) {
     using Mm = Mma<PREC>;
     using frag = typename Mm::frag;
     using P = ShadeLds<PREC>;
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     };
     const size_t w1 = L.w1 + (size_t)wave * T1 * NP * LM_WAVE * sizeof(frag), w2 = L.w2 + (size_t)wave * T2 * NP * LM_WAVE * sizeof(frag);
     auto bias_of = [&](size_t at, uint32_t half) { return load_bias(reinterpret_cast<const float *>(packed + at + half), 0); };
-    const uint32_t M = min(*count, cap);  // the counter keeps counting past the list's capacity
+    const uint32_t M = FEAT ? M_host : min(*count, cap);  // the counter keeps counting past the list's capacity
     const uint32_t n_tiles = (uint32_t)(((uint64_t)M + kTileRays - 1) / kTileRays);
     // Workgroup b runs on XCD b % 8: granules of four neighbouring tiles stay on one XCD and share its L2
     uint32_t b = blockIdx.x;
@@ -135,9 +136,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         return acc;
     };
     if (b >= n_tiles) return;
-    auto entry = [&](uint32_t tile, uint32_t i) { return list[min((uint64_t)tile * kTileRays + i, (uint64_t)M - 1u)]; };
+    auto entry = [&](uint32_t tile, uint32_t i) {
+        const uint32_t at = (uint32_t)min((uint64_t)tile * kTileRays + i, (uint64_t)M - 1u);
+        return FEAT ? at : list[at];
+    };
     float q[4], vnext[3];  // coordinates of the lane's sample and its column's view direction
     auto position = [&](uint32_t gather, uint32_t column) {
+        if constexpr (FEAT) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) q[i] = rays[3 * (size_t)gather + i];
+            q[3] = 0.0f;
+            return;
+        }
         list_coords(g, rays, gather, q);
         const float *d = rays + 6 * (size_t)(column / (uint32_t)g.S) + 3;
 #pragma unroll
@@ -194,7 +204,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         }
         // the wave's weights of layer 1 travel while basis_mat is applied
         frag wa[T1][NP];
-        constexpr int kFirst = G == 1 || NP == 2 ? T1 / 2 : T1;  // the rest once basis_mat's fragments have left the registers
+        constexpr int kFirst = FEAT ? 0 : G == 1 || NP == 2 ? T1 / 2 : T1;  // the rest once basis_mat's fragments have left the registers
 #pragma unroll
         for (int t = 0; t < kFirst; ++t)
 #pragma unroll
@@ -237,8 +247,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 if (k + 2 < ps.n) request(k + 2, a0);
                 if (k + 1 < ps.n) multiply(k + 1, a1);
             }
+            if constexpr (FEAT) {
+                const uint32_t p = tile * kTileRays + j;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) raw_s[v * LM_WAVE + lane] = acc[v];
+                for (int v = 0; v < 16; ++v)
+                    if (p < M && row_of(v, (int)h) < kAppDim) rgb[(size_t)p * kAppDim + row_of(v, (int)h)] = acc[v];
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) raw_s[v * LM_WAVE + lane] = acc[v];
+            }
+        }
+        if constexpr (FEAT) {
+            position(gn, vn);
+            __syncthreads();  // the next tile's products overwrite this one's
+            continue;
         }
         acc = bias_of(L.b1 + wave * 128u, bias);
 #pragma unroll
@@ -343,11 +365,11 @@ size_t shade_lds(int prec, int K) {
     }
 }
 
-template <int PREC, typename T, int NU>
-int launch_shade(const lm_model *m, int K, const float *rays, const uint32_t *list, const uint32_t *count, uint32_t cap, float *rgb,
-                 hipStream_t st) {
+template <int PREC, typename T, int NU, bool FEAT>
+int launch_shade(const lm_geom &geom, const PlaneSet &ps, int K, const void *packed, const float *rays, uint32_t M, const uint32_t *list,
+                 const uint32_t *count, uint32_t cap, float *rgb, hipStream_t st) {
     const size_t lds = ShadeLds<PREC>::total(K);
-    auto kern = &k_shade<PREC, T, NU>;
+    auto kern = &k_shade<PREC, T, NU, FEAT>;
     static thread_local size_t reserved_on[LM_MAX_DEVICES] = {};  // set once per thread, device, kernel, size
     size_t &reserved = reserved_on[lm_current_device()];
     if (reserved != lds) {
@@ -355,11 +377,41 @@ int launch_shade(const lm_model *m, int K, const float *rays, const uint32_t *li
         if (e != hipSuccess) LM_FAIL(LM_ERR_LAUNCH, "k_shade: LDS reservation failed: %s", hipGetErrorString(e));
         reserved = lds;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)lm_persistent_blocks(2)), dim3(kBlock), lds, st, m->geom,
-                       make_set(m->app, m->n_planes, &m->geom), K, (const char *)m->mlp_packed, pack_layout(PREC, K), rays, list, count,
-                       cap, rgb);
+    unsigned grid = (unsigned)lm_persistent_blocks(2);
+    if (FEAT) grid = std::min(grid, (M + kTileRays - 1) / kTileRays);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, st, geom, ps, K, (const char *)packed, pack_layout(PREC, K), rays, M, list,
+                       count, cap, rgb);
     LM_CHECK_LAUNCH("k_shade");
     return LM_OK;
+}
+
+template <bool FEAT>
+int shade(int prec, int dtype, int nu, const lm_geom &geom, const PlaneSet &ps, int K, const void *packed, const float *rays, uint32_t M,
+          const uint32_t *list, const uint32_t *count, uint32_t cap, float *rgb, hipStream_t st) {
+#define LM_SHADE_NU(PREC_, T_, NU_) launch_shade<PREC_, T_, NU_, FEAT>(geom, ps, K, packed, rays, M, list, count, cap, rgb, st)
+#define LM_SHADE(PREC_)                                              \
+    if (dtype == LM_F32) {                                           \
+        switch (nu) {                                                \
+            case 1: return LM_SHADE_NU(PREC_, float, 1);             \
+            case 2: return LM_SHADE_NU(PREC_, float, 2);             \
+            case 3: return LM_SHADE_NU(PREC_, float, 3);             \
+            default: return LM_SHADE_NU(PREC_, float, 4);            \
+        }                                                            \
+    }                                                                \
+    switch (nu) {                                                    \
+        case 1: return LM_SHADE_NU(PREC_, Half4, 1);                 \
+        case 2: return LM_SHADE_NU(PREC_, __half, 2);                \
+        case 3: return LM_SHADE_NU(PREC_, Half6, 3);                 \
+        default: return LM_SHADE_NU(PREC_, __half, 4);               \
+    }
+    switch (prec) {
+        case LM_MLP_F32: LM_SHADE(LM_MLP_F32)
+        case LM_MLP_F16: LM_SHADE(LM_MLP_F16)
+        case LM_MLP_BF16: LM_SHADE(LM_MLP_BF16)
+        default: LM_SHADE(LM_MLP_F16X2)
+    }
+#undef LM_SHADE
+#undef LM_SHADE_NU
 }
 
 }  // namespace
@@ -382,6 +434,14 @@ bool lm_shade_takes(const lm_model *m, int64_t N, int K) {
     return shade_covers(m, K) && N * m->geom.S <= (m->mlp_prec == LM_MLP_F32 ? 1ll << 19 : 3ll << 20);
 }
 
+// compute_appfeature at given points: up to here a tile per workgroup beats k_app_feat's tile per wave.  Nine planes, split
+// mode, products through memory / k_app_feat / here: 4000 points 38 / 51 / 16 us, 32000: 75 / 75 / 50, 64000: 150 / 84 / 95;
+// fp16 mode (k_app_feat has two workgroups per CU there): 32000: 74 / 124 / 47, 64000: 148 / 151 / 88, 128000: 304 / 161 / 173.
+bool lm_few_points_take(int prec, int K, int64_t M) {
+    const int64_t limit = prec == LM_MLP_F16 || prec == LM_MLP_BF16 ? 96 * 1024 : 48 * 1024;
+    return M <= limit && shade_lds(prec, K) <= 80 * 1024;
+}
+
 // `count` list entries (at most `cap`) -> rgb [count, 3]; what lm_launch_app_features + lm_launch_app_colour give.
 int lm_launch_shade(const lm_model *m, const float *rays, const uint32_t *list, const uint32_t *count, uint32_t cap, float *rgb,
                     hipStream_t st) {
@@ -392,29 +452,12 @@ int lm_launch_shade(const lm_model *m, const float *rays, const uint32_t *list, 
     LM_REQUIRE(rays && list && count && rgb, "null buffer");
     LM_REQUIRE(m->mlp_packed && lm_aligned16(m->mlp_packed), "packed colour-network weights are null or misaligned");
     if (!shade_covers(m, K)) LM_FAIL(LM_ERR_UNSUPPORTED, "k_shade does not cover these planes");
-    const int nu = m->app[0].C / 16;
-#define LM_SHADE_NU(PREC_, T_, NU_) launch_shade<PREC_, T_, NU_>(m, K, rays, list, count, cap, rgb, st)
-#define LM_SHADE(PREC_)                                              \
-    if (dtype == LM_F32) {                                           \
-        switch (nu) {                                                \
-            case 1: return LM_SHADE_NU(PREC_, float, 1);             \
-            case 2: return LM_SHADE_NU(PREC_, float, 2);             \
-            case 3: return LM_SHADE_NU(PREC_, float, 3);             \
-            default: return LM_SHADE_NU(PREC_, float, 4);            \
-        }                                                            \
-    }                                                                \
-    switch (nu) {                                                    \
-        case 1: return LM_SHADE_NU(PREC_, Half4, 1);                 \
-        case 2: return LM_SHADE_NU(PREC_, __half, 2);                \
-        case 3: return LM_SHADE_NU(PREC_, Half6, 3);                 \
-        default: return LM_SHADE_NU(PREC_, __half, 4);               \
-    }
-    switch (m->mlp_prec) {
-        case LM_MLP_F32: LM_SHADE(LM_MLP_F32)
-        case LM_MLP_F16: LM_SHADE(LM_MLP_F16)
-        case LM_MLP_BF16: LM_SHADE(LM_MLP_BF16)
-        default: LM_SHADE(LM_MLP_F16X2)
-    }
-#undef LM_SHADE
-#undef LM_SHADE_NU
+    return shade<false>(m->mlp_prec, dtype, m->app[0].C / 16, m->geom, make_set(m->app, m->n_planes, &m->geom), K, m->mlp_packed, rays,
+                        0u, list, count, cap, rgb, st);
+}
+
+// M points (M < 2^31) -> feat [M, 27]; the caller has checked the arguments and asked lm_few_points_take
+int lm_launch_few_points(const lm_plane *planes, int n, int prec, int dtype, int K, const void *packed, const float *xyz, uint32_t M,
+                         float *feat, hipStream_t st) {
+    return shade<true>(prec, dtype, planes[0].C / 16, lm_geom{}, make_set(planes, n), K, packed, xyz, M, nullptr, nullptr, 0u, feat, st);
 }

@@ -1,7 +1,8 @@
 """The back half of a render has two forms: one kernel per stage (large chunks) and one kernel from appearance entries to
 colours (small chunks).  Both do the same operations in the same order, so pictures agree exactly, in every arithmetic mode
 and for every channel width, storage type and number of planes the small form covers; widths and mixtures it does not cover
-take the kernels per stage.  compute_appfeature has the same two forms: one kernel, and products through memory."""
+take the kernels per stage.  compute_appfeature has both forms too (few and many points), and
+a third one through memory for what they do not cover."""
 import pytest
 import torch
 
@@ -45,7 +46,7 @@ def test_appearance_features_of_points_equal_products_and_projection(gpu_lib, ne
 
     m = GridNeRFHIP(_scene(an, ndims, res, fp16), device="cuda", mlp_precision=net)
     g = torch.Generator().manual_seed(3)
-    for n in (1, 31, 32, 33, 5000):
+    for n in (1, 31, 32, 33, 5000, 99001):  # a tile per workgroup, several of them, a tile per wave
         xyz = torch.rand((n, 3), generator=g) * 2.6 - 1.3  # some outside the tables
         xyz[0] = float("nan")
         got = m.compute_appfeature(xyz)
