@@ -143,7 +143,9 @@ typedef struct lm_model {
     int32_t mlp_prec;   /* LM_MLP_* the packed weights were packed for */
     const void *mlp_packed; /* device copy of the buffer written by lm_mlp_pack */
     int32_t white_bg;
-    float term_eps; /* > 0: stop marching a ray once transmittance < term_eps */
+    float term_eps; /* > 0: stop marching a ray once transmittance < term_eps.  0: gather every valid sample.  < 0: stop
+                     * where no later sample can change opacity, depth or the appearance list, same bits as 0; the caller
+                     * promises finite tables (a NaN behind that point would not be seen) and a positive distance_scale */
     /* Hint: the chunk's rays are the pixels of an image stored row by row, ray_row of them per
      * row (the chunk may start anywhere in a row).  lm_render then visits rays in 8 x 8 pixel
      * tiles, so that rays handled together are neighbours in both directions and share more of
@@ -188,6 +190,11 @@ const char *lm_last_error(void);
  * out channel-last the same way (app/models/gridnerf_elastic_cuda.py:274-303). */
 int lm_relayout_nchw_to_hwc(const void *src, void *dst, int32_t C, int32_t H, int32_t W, int32_t dtype,
                             void *stream);
+/* The same, and the largest magnitudes of the table's parts: writes lm_relayout_peak_words() words at `peak` (device memory,
+ * may be NULL), whose maximum holds the bits of max |x| (fp16 bits for an fp16 table; above those of infinity when the
+ * table holds a NaN). */
+size_t lm_relayout_peak_words(int32_t C, int32_t H, int32_t W);
+int lm_relayout_peak(const void *src, void *dst, int32_t C, int32_t H, int32_t W, int32_t dtype, uint32_t *peak, void *stream);
 
 /* Build the cell table of a 0/1 occupancy volume (float [D][H][W]); *not_binary (device
  * uint32, zeroed by the caller) is set to 1 if a voxel is neither 0 nor 1, in which case the

@@ -60,6 +60,8 @@ SYMBOLS = {
     "lm_abi_version": (C.c_int, []),
     "lm_last_error": (C.c_char_p, []),
     "lm_relayout_nchw_to_hwc": (C.c_int, [_P, _P, _I32, _I32, _I32, _I32, _P]),
+    "lm_relayout_peak_words": (_SZ, [_I32, _I32, _I32]),
+    "lm_relayout_peak": (C.c_int, [_P, _P, _I32, _I32, _I32, _I32, _P, _P]),
     "lm_pack_occupancy": (C.c_int, [_P, _I32, _I32, _I32, _P, _P, _P]),
     "lm_occupancy_coarse_bytes": (_SZ, [_I32, _I32, _I32]),
     "lm_pack_occupancy_coarse": (C.c_int, [_P, _I32, _I32, _I32, _P, _P]),

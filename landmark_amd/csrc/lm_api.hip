@@ -36,17 +36,30 @@ int lm_persistent_blocks(int blocks_per_cu) {
 
 // ---- [C,H,W] -> [H,W,C] ---------------------------------------------------------------------
 namespace {
+__device__ __forceinline__ uint32_t magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+__device__ __forceinline__ uint32_t magnitude(uint16_t half) { return half & 0x7fffu; }
+
 template <typename T>
-__global__ __launch_bounds__(256) void k_relayout(const T *__restrict__ src, T *__restrict__ dst, int C, uint64_t HW) {
+__global__ __launch_bounds__(256) void k_relayout(const T *__restrict__ src, T *__restrict__ dst, int C, uint64_t HW, uint32_t *peak) {
     // 64 texels x 64 channels per tile through LDS: coalesced reads along HW, coalesced writes along C
     __shared__ T tile[64][65];
     const uint64_t t0 = (uint64_t)blockIdx.x * 64;
     const int c0 = blockIdx.y * 64;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    uint32_t top = 0;  // largest magnitude as bits: ordered like the magnitudes, infinities and NaNs above all numbers
     for (int cc = ty; cc < 64; cc += 4) {
         const int c = c0 + cc;
         const uint64_t t = t0 + tx;
-        if (c < C && t < HW) tile[cc][tx] = src[(uint64_t)c * HW + t];
+        if (c < C && t < HW) {
+            const T v = src[(uint64_t)c * HW + t];
+            tile[cc][tx] = v;
+            top = max(top, magnitude(v));
+        }
+    }
+    if (peak) {
+#pragma unroll
+        for (int d = 1; d < LM_WAVE; d <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d));
+        if (tx == 0) peak[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + ty] = top;
     }
     __syncthreads();
     for (int tt = ty; tt < 64; tt += 4) {
@@ -59,6 +72,16 @@ __global__ __launch_bounds__(256) void k_relayout(const T *__restrict__ src, T *
 
 extern "C" int lm_relayout_nchw_to_hwc(const void *src, void *dst, int32_t C, int32_t H, int32_t W, int32_t dtype,
                                        void *stream) {
+    return lm_relayout_peak(src, dst, C, H, W, dtype, nullptr, stream);
+}
+
+extern "C" size_t lm_relayout_peak_words(int32_t C, int32_t H, int32_t W) {
+    if (C <= 0 || H <= 0 || W <= 0) return 0;
+    return ((size_t)H * W + 63) / 64 * (((size_t)C + 63) / 64) * 4;  // a word per wave: no atomics, no contention
+}
+
+extern "C" int lm_relayout_peak(const void *src, void *dst, int32_t C, int32_t H, int32_t W, int32_t dtype, uint32_t *peak,
+                                void *stream) {
     LM_REQUIRE(src && dst && src != dst, "null or aliased buffer");
     LM_REQUIRE(C > 0 && H > 0 && W > 0, "empty table");
     LM_REQUIRE(dtype == LM_F32 || dtype == LM_F16, "unknown dtype %d", dtype);
@@ -67,10 +90,11 @@ extern "C" int lm_relayout_nchw_to_hwc(const void *src, void *dst, int32_t C, in
     LM_REQUIRE(bx < (1ull << 31), "table too large");
     dim3 grid((unsigned)bx, (unsigned)((C + 63) / 64));
     if (dtype == LM_F32)
-        hipLaunchKernelGGL(k_relayout<float>, grid, dim3(256), 0, (hipStream_t)stream, (const float *)src, (float *)dst, C, HW);
+        hipLaunchKernelGGL(k_relayout<float>, grid, dim3(256), 0, (hipStream_t)stream, (const float *)src, (float *)dst, C, HW,
+                           peak);
     else
         hipLaunchKernelGGL(k_relayout<uint16_t>, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t *)src,
-                           (uint16_t *)dst, C, HW);
+                           (uint16_t *)dst, C, HW, peak);
     LM_CHECK_LAUNCH("k_relayout");
     return LM_OK;
 }

@@ -138,7 +138,8 @@ __global__ __launch_bounds__(kBlock) void k_app_list(lm_geom g, PlaneSet ps, int
 // stay busy whatever the rays' lengths.  Two things follow from walking rays in lock step:
 // neighbouring rays are at similar depths in the same load instruction, so their corner
 // texels share cache lines; and a ray can stop once its transmittance is below term_eps,
-// before the density of the samples behind is ever fetched.  With term_eps = 0 the weights
+// before the density of the samples behind is ever fetched, or (term_eps < 0) once nothing behind can change its results
+// (155.8 -> 135 million samples gathered for 518400 rays of 3544 steps, 8.4 -> 6.2 million for 160000 rays of 128).  With term_eps = 0 the weights
 // are those of the separate density + weights kernels, bit for bit (same operations, and the
 // transmittance is the same sequential product torch.cumprod forms, app/tools/utils.py:51-64).
 template <typename T, int NS>  // NS samples of a ray per round
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
     bool have = false, done = false;
     uint32_t r = 0, p = 0, cnt = 0;
     uint64_t flat0 = 0;
-    float ray[6] = {0, 0, 0, 0, 0, 0}, rp = 0.0f, Tr = 1.0f, acc = 0.0f, depth = 0.0f;
+    float ray[6] = {0, 0, 0, 0, 0, 0}, rp = 0.0f, Tr = 1.0f, acc = 0.0f, depth = 0.0f, z_last = 0.0f;
     BitWalk it;
     it.bits = 0; it.w = it.w0 = it.w_last = 0; it.flat1 = 0; it.pos = 0; it.bitmap = bitmap; it.prefix = nullptr;
     it.todo = it.ahead = 0; it.masked = false;
@@ -201,6 +202,7 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
                     flat0 = (uint64_t)r * (uint64_t)S;
                     it.start_at(bitmap, flat0, flat0 + S, p_first[r], word_mask ? word_mask[r] : ~0ull);
                     p = it.pos;
+                    z_last = lm_sample_z(g, rp, S - 1);
                     Tr = 1.0f; acc = 0.0f; depth = 0.0f; cnt = 0;
                     have = true;
                 }
@@ -264,6 +266,8 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
                     finish = term_eps > 0.0f && Tr < term_eps;
                 }
                 if (n_have < NS) finish = true;  // the ray's last samples
+                else if (term_eps < 0.0f && !finish)
+                    finish = lm_rest_is_lost(Tr, acc, depth, quad_lane(dist, NS - 1), z_last, weight_thres);
             }
             if (finish) {
                 if (qlane == 0) {

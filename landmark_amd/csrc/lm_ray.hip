@@ -18,7 +18,8 @@
 // samples of a round do not fill the waves (4096 rays of 128 samples on nine planes: 82 / 58 / 80 / 133 us with 8 / 4 / 2 /
 // 1 rays before the transmittance was spread over the lanes).
 // Measured against zeroed bitmap + cull + march with a wave per ray + list: 4096 rays as above 93 -> 45 us, 8192 rays of
-// 886 samples on three planes 393 -> 310 us, 1024 rays on three 256^2 planes 51 -> 23 us.
+// 886 samples on three planes 393 -> 310 us, 1024 rays on three 256^2 planes 51 -> 23 us.  With term_eps < 0 (rays
+// stop after the round behind which nothing can change their results) the second takes 229 us, the third 20.
 // Operations and order per ray are those of the kernels for large chunks, hence the same bits.
 #include <algorithm>
 
@@ -288,6 +289,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 }
             }
             if (over) left = 0u;
+            else if (term_eps < 0.0f && left) {
+                auto of = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+                const float z_last = lm_sample_z(g, s_ray[wave][6], S - 1), dist = z_last - of(z_m, 0);
+                if (lm_rest_is_lost(of(Tr, 0), of(sum, 0), of(sum, 1), dist / (float)S, z_last, weight_thres)) left = 0u;
+            }
             const bool take = w_m > weight_thres && lane < used;
             const uint64_t bits = __ballot(take);
             const uint32_t cnt = s_cnt[wave], slot = cnt + lm_mbcnt(bits);

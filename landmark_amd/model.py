@@ -12,6 +12,7 @@ library, or without a GPU, construction raises.
 from __future__ import annotations
 
 import ctypes as C
+import math
 from types import SimpleNamespace
 from typing import Dict, Optional, Tuple
 
@@ -101,7 +102,8 @@ class GridNeRFHIP:
                 raise L.LandmarkError("plane_division [1, 1]: one block is the plain layout; squeeze the block axis "
                                       "(planes [1,C,h,w], lines [1,C,L,1]) and pass plane_division=None")
         self._tables = []  # keep device tensors alive
-        self._density = self._relayout_set(params.density_plane, params.density_line)
+        peaks = []
+        self._density = self._relayout_set(params.density_plane, params.density_line, peaks)
         self._app = self._relayout_set(params.app_plane, params.app_line)
         self.K_app = sum(pl.C for pl in self._app)
         if release_source:
@@ -112,6 +114,8 @@ class GridNeRFHIP:
             self._den_w = params.basis_den.detach().to(self.device, torch.float32).reshape(-1).contiguous()
             if self._den_w.numel() != sum(pl.C for pl in self._density):
                 raise L.LandmarkError("basis_den width does not match the density planes")
+        # rays may stop where the rest cannot change their results (lm_model.term_eps < 0) if the densities are finite
+        self._finite_densities = self._density_bound(torch.stack(peaks).cpu().numpy()) < 1e30 and 0.0 < float(params.distance_scale) < 1e30
         # --- colour network; with encode_app the 48 latent columns of the first layer fold into its bias
         self.encode_app = bool(params.encode_app)
         self._latent_dim = 0
@@ -179,17 +183,22 @@ class GridNeRFHIP:
                 if bool((as_u8.float() == self._vol).all()):
                     self._vol_dtype, self._vol_store = L.LM_U8, as_u8.contiguous()
 
-    def _relayout(self, t: torch.Tensor) -> torch.Tensor:
-        """[1,C,H,W] -> device [H,W,C] through lm_relayout_nchw_to_hwc."""
+    def _relayout(self, t: torch.Tensor, peaks: Optional[list] = None) -> torch.Tensor:
+        """[1,C,H,W] -> device [H,W,C] through lm_relayout_peak; the bits of max |t| (one device word) go to `peaks`."""
         src = t.to(self.device).contiguous()
         _, Cc, H, W = src.shape
         dst = torch.empty((H, W, Cc), dtype=src.dtype, device=self.device)
         dt = L.LM_F32 if src.dtype == torch.float32 else L.LM_F16
-        L.check(self.lib.lm_relayout_nchw_to_hwc(src.data_ptr(), dst.data_ptr(), Cc, H, W, dt, L.current_stream()), "relayout")
+        peak = None
+        if peaks is not None:
+            peak = torch.empty(self.lib.lm_relayout_peak_words(Cc, H, W), dtype=torch.int32, device=self.device)
+        L.check(self.lib.lm_relayout_peak(src.data_ptr(), dst.data_ptr(), Cc, H, W, dt, L.ptr(peak), L.current_stream()), "relayout")
+        if peaks is not None:
+            peaks.append(peak.max())
         torch.cuda.current_stream().synchronize()  # src may be a temporary
         return dst
 
-    def _relayout_set(self, planes, lines):
+    def _relayout_set(self, planes, lines, peaks=None):
         out = []
         L_ = len(self.resMode)
         if len(planes) > L.LM_MAX_PLANES:
@@ -203,12 +212,12 @@ class GridNeRFHIP:
                 if pl.dim() != 5 or pl.shape[2] != self._n_blocks or ln.shape[-1] != self._n_blocks:
                     raise L.LandmarkError(f"plane {k}: shapes {tuple(pl.shape)}, {tuple(ln.shape)} do not hold {self._n_blocks} blocks")
                 _, Cc, B, h, w = pl.shape
-                P, Ln = self._relayout(pl.reshape(1, Cc, B * h, w)), self._relayout(ln)
+                P, Ln = self._relayout(pl.reshape(1, Cc, B * h, w), peaks), self._relayout(ln, peaks)
                 s.H, s.W, s.C = h, w, Cc
             else:
                 if pl.dim() != 4:
                     raise L.LandmarkError(f"plane {k} has shape {tuple(pl.shape)}: block-stacked planes need plane_division")
-                P, Ln = self._relayout(pl), self._relayout(ln)
+                P, Ln = self._relayout(pl, peaks), self._relayout(ln, peaks)
                 s.H, s.W, s.C = P.shape
             self._tables += [P, Ln]
             d = k // L_
@@ -219,6 +228,18 @@ class GridNeRFHIP:
             s.dtype = L.LM_F32 if P.dtype == torch.float32 else L.LM_F16
             out.append(s)
         return out
+
+    def _density_bound(self, peaks) -> float:
+        """Upper bound of |density feature| over all points (inf where a table holds a NaN or an infinity), from the
+        bits of the largest magnitudes, one word per table (plane, line, plane, ...)."""
+        bound = 0.0
+        for pl, words in zip(self._density, peaks.reshape(-1, 2)):
+            top = words.view(np.float32) if pl.dtype == L.LM_F32 else words.astype(np.uint16).view(np.float16)
+            bound += pl.C * float(top[0]) * float(top[1])
+        if self._den_w is not None:
+            bound *= float(self._den_w.abs().max())
+        bound += abs(float(self.p.density_shift))
+        return bound if math.isfinite(bound) else math.inf
 
     FP16_MAX = 65504.0
 
@@ -361,7 +382,7 @@ class GridNeRFHIP:
         """The lm_model of a render with S samples per ray and workspace capacities `caps` (valid samples,
         appearance samples; 0 = worst case), built once per distinct setting and reused (a caller that keeps
         small chunks pays for launches only); never carries event handles."""
-        key = (int(S), bool(white_bg), self.mlp_precision, float(self.term_eps), int(self.ray_row_length), caps)
+        key = (int(S), bool(white_bg), self.mlp_precision, float(self.term_eps), self._finite_densities, int(self.ray_row_length), caps)
         m = self._struct_cache.get(key)
         if m is None:
             if len(self._struct_cache) > 64:
@@ -385,7 +406,8 @@ class GridNeRFHIP:
         prec, packed = self._pack_mlp(self.mlp_precision)
         m.mlp_prec, m.mlp_packed = prec, packed.data_ptr()
         m.white_bg = int(bool(white_bg))
-        m.term_eps = self.term_eps
+        # exact results asked for: a ray may still stop once nothing behind can change them (finite densities only)
+        m.term_eps = self.term_eps if self.term_eps > 0 else (-1.0 if self._finite_densities else 0.0)
         m.ray_row = int(self.ray_row_length)
         return m
 
