@@ -111,6 +111,7 @@ int lm_launch_app_products(const lm_model *m, const float *rays, const uint32_t 
                            float *products, hipStream_t st);
 int lm_launch_composite(int64_t N, const uint32_t *app_first, const uint32_t *app_cnt, const float *app_w,
                         const float *rgb, const float *acc, int white_bg, uint32_t row, float *rgb_map,
+                        const uint32_t *ray_valid, const uint32_t *ray_marched, int count_valid, uint32_t *counters,
                         hipStream_t stream);
 int lm_launch_zero_counters(uint32_t *counters, hipStream_t stream);
 int lm_launch_cull_setup(const lm_geom *geom, const float *rays, int64_t N, uint64_t *bitmap, uint32_t *p_first,
@@ -128,7 +129,7 @@ int lm_launch_march(const lm_model *m, const float *rays, const uint64_t *bitmap
 bool lm_rays_kernel_takes(const lm_model *m, int64_t N);
 int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t row, uint32_t cap_valid, uint32_t *app_first,
                    uint32_t *app_cnt, uint32_t *app_idx, float *app_w, uint32_t cap_app, float *acc, float *depth,
-                   uint32_t *counters, hipStream_t st);
+                   uint32_t *ray_valid, uint32_t *ray_marched, uint32_t *counters, hipStream_t st);
 bool lm_shade_takes(const lm_model *m, int64_t N, int K);
 int lm_launch_shade(const lm_model *m, const float *rays, const uint32_t *list, const uint32_t *count, uint32_t cap, float *rgb,
                     hipStream_t st);
@@ -302,9 +303,9 @@ int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *w
     if (int rc = lm_launch_zero_counters(cnt, st)) return rc;
     const bool few = lm_rays_kernel_takes(m, N);
     if (few) {
-        // few rays: one kernel up to the appearance list
+        // few rays: one kernel up to the appearance list (p_first, p_end: samples valid and gathered per ray)
         if (int rc = lm_launch_rays(m, rays, (uint32_t)N, row, (uint32_t)w.cap_valid, w.app_first, w.app_cnt, w.app_idx, w.app_w,
-                                    (uint32_t)w.cap_app, w.acc, depth_map, cnt, st))
+                                    (uint32_t)w.cap_app, w.acc, depth_map, w.p_first, w.p_end, cnt, st))
             return rc;
         mark(LM_STAGE_CULL);
         mark(LM_STAGE_DENSITY);
@@ -346,7 +347,11 @@ int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *w
             return rc;
     }
     mark(LM_STAGE_COLOUR);
-    if (int rc = lm_launch_composite(N, w.app_first, w.app_cnt, w.app_w, w.rgb, w.acc, m->white_bg, row, rgb_map, st)) return rc;
+    // k_rays has counted the valid samples itself where it had to check them against a capacity
+    const int count_valid = w.cap_valid >= (uint64_t)N * (uint64_t)S;
+    if (int rc = lm_launch_composite(N, w.app_first, w.app_cnt, w.app_w, w.rgb, w.acc, m->white_bg, row, rgb_map, few ? w.p_first : nullptr,
+                                     few ? w.p_end : nullptr, count_valid, cnt, st))
+        return rc;
     mark(LM_STAGE_COMPOSITE);
     return LM_OK;
 }

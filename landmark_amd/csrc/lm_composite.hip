@@ -110,39 +110,64 @@ __global__ __launch_bounds__(kBlock) void k_weights(lm_geom g, const float *__re
     }
 }
 
+// Samples per ray (any order) and where their sums go; count_valid: whether the valid ones are not counted there already
+struct RayStats {
+    const uint32_t *valid, *marched;
+    uint32_t *counters;
+    int count_valid;
+};
+
 // A quad per ray, a lane per colour channel: a quad's loads fall into one run of the list whatever the order the rays'
 // ranges lie in, sixteen entries in flight.  A lane per ray, with the wave's range of the list staged through LDS in
 // windows, waits for each window and does badly where neighbouring rays' ranges lie apart (k_rays reserves four rays at a
 // time): 8192 rays of 30 entries 13 - 75 -> 5.8 us, 4096 rays of 5 entries 13 -> 5 us, 518400 rays of 57 entries 390 -> 223 us,
 // a million rays of 11 entries 74 us either way.  Eight entries in flight: 7.1, 5.1, 279, 81 us.
+// STATS: the idle lane of every quad also takes its ray's sample counts, which k_rays leaves per ray, and the workgroup
+// adds the sums to the counter block.
+template <bool STATS>
 __global__ __launch_bounds__(kBlock) void k_composite(uint64_t N, const uint32_t *__restrict__ app_first,
                                                            const uint32_t *__restrict__ app_cnt, const float *__restrict__ app_w,
                                                            const float *__restrict__ rgb, const float *__restrict__ acc, int white_bg,
-                                                           uint32_t row, float *__restrict__ rgb_map) {
+                                                           uint32_t row, float *__restrict__ rgb_map, RayStats stats) {
     const uint64_t o = (uint64_t)blockIdx.x * (kBlock / 4) + threadIdx.x / 4;
     const unsigned ch = threadIdx.x & 3u;
-    if (o >= N || ch == 3u) return;
-    const uint64_t r = lm_ray_order((uint32_t)o, (uint32_t)N, row);
-    constexpr uint32_t kAhead = 16;
-    const uint32_t n = app_cnt[r];
-    const size_t first = app_first[r];
-    const float a = white_bg ? acc[r] : 0.0f;
-    const float *w = app_w + first, *c = rgb + 3 * first + ch;
-    float sum = 0.0f;
-    for (uint32_t i = 0; i < n; i += kAhead) {
-        float wv[kAhead], cv[kAhead];
-#pragma unroll
-        for (uint32_t u = 0; u < kAhead; ++u) {
-            const uint32_t at = min(i + u, n - 1u);
-            wv[u] = w[at];
-            cv[u] = c[3 * (size_t)at];
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kAhead; ++u)
-            if (i + u < n) sum = fmaf(wv[u], cv[u], sum);
+    __shared__ uint32_t s_sum[2];
+    uint32_t n_valid = 0, n_marched = 0;
+    if constexpr (STATS) {
+        if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+        if (o < N && ch == 3u) { n_valid = stats.valid[o]; n_marched = stats.marched[o]; }
     }
-    if (white_bg) sum += 1.0f - a;
-    rgb_map[3 * r + ch] = fminf(fmaxf(sum, 0.0f), 1.0f);
+    if (o < N && ch != 3u) {
+        const uint64_t r = lm_ray_order((uint32_t)o, (uint32_t)N, row);
+        constexpr uint32_t kAhead = 16;
+        const uint32_t n = app_cnt[r];
+        const size_t first = app_first[r];
+        const float a = white_bg ? acc[r] : 0.0f;
+        const float *w = app_w + first, *c = rgb + 3 * first + ch;
+        float sum = 0.0f;
+        for (uint32_t i = 0; i < n; i += kAhead) {
+            float wv[kAhead], cv[kAhead];
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u) {
+                const uint32_t at = min(i + u, n - 1u);
+                wv[u] = w[at];
+                cv[u] = c[3 * (size_t)at];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u)
+                if (i + u < n) sum = fmaf(wv[u], cv[u], sum);
+        }
+        if (white_bg) sum += 1.0f - a;
+        rgb_map[3 * r + ch] = fminf(fmaxf(sum, 0.0f), 1.0f);
+    }
+    if constexpr (STATS) {
+        __syncthreads();
+        if (n_valid) atomicAdd(&s_sum[0], n_valid);
+        if (n_marched) atomicAdd(&s_sum[1], n_marched);
+        __syncthreads();
+        if (threadIdx.x == 0 && stats.count_valid && s_sum[0]) atomicAdd(stats.counters + LM_STAT_N_VALID, s_sum[0]);
+        if (threadIdx.x == 1 && s_sum[1]) atomicAdd(stats.counters + LM_STAT_N_MARCHED, s_sum[1]);
+    }
 }
 
 // Appearance list from stored weights: a contiguous slot range per ray (wave prefix + one
@@ -260,10 +285,17 @@ extern "C" int lm_weights(const lm_geom *geom, const float *rays, int64_t N, con
 
 int lm_launch_composite(int64_t N, const uint32_t *app_first, const uint32_t *app_cnt, const float *app_w,
                         const float *rgb, const float *acc, int white_bg, uint32_t row, float *rgb_map,
+                        const uint32_t *ray_valid, const uint32_t *ray_marched, int count_valid, uint32_t *counters,
                         hipStream_t stream) {
     if (N == 0) return LM_OK;
-    hipLaunchKernelGGL(k_composite, dim3((unsigned)(((uint64_t)N + kBlock / 4 - 1) / (kBlock / 4))), dim3(kBlock), 0, stream,
-                       (uint64_t)N, app_first, app_cnt, app_w, rgb, acc, white_bg, row, rgb_map);
+    const RayStats stats = {ray_valid, ray_marched, counters, count_valid};
+    const dim3 grid((unsigned)(((uint64_t)N + kBlock / 4 - 1) / (kBlock / 4)));
+    if (ray_valid)
+        hipLaunchKernelGGL(k_composite<true>, grid, dim3(kBlock), 0, stream, (uint64_t)N, app_first, app_cnt, app_w, rgb, acc, white_bg,
+                           row, rgb_map, stats);
+    else
+        hipLaunchKernelGGL(k_composite<false>, grid, dim3(kBlock), 0, stream, (uint64_t)N, app_first, app_cnt, app_w, rgb, acc, white_bg,
+                           row, rgb_map, stats);
     LM_CHECK_LAUNCH("k_composite");
     return LM_OK;
 }
@@ -274,7 +306,8 @@ extern "C" int lm_composite_rgb(int64_t N, const uint32_t *app_first, const uint
     if (N == 0) return LM_OK;
     LM_REQUIRE((uint64_t)N < (1ull << 32), "ray count does not fit 32 bits");
     LM_REQUIRE(app_first && app_cnt && app_w && rgb && acc && rgb_map, "null buffer");
-    return lm_launch_composite(N, app_first, app_cnt, app_w, rgb, acc, white_bg, 0u, rgb_map, (hipStream_t)stream);
+    return lm_launch_composite(N, app_first, app_cnt, app_w, rgb, acc, white_bg, 0u, rgb_map, nullptr, nullptr, 0, nullptr,
+                               (hipStream_t)stream);
 }
 
 int lm_launch_zero_counters(uint32_t *counters, hipStream_t stream) {

@@ -13,7 +13,10 @@
 //      samples that are usual at 128 samples per ray;
 //   3. the transmittance runs through a ray's samples of the round in order (the product torch.cumprod forms); the
 //      round's appearance entries are appended to the ray's list in LDS;
-//   4. one reservation per workgroup in the appearance list.
+//   4. one reservation per workgroup in the appearance list.  It is the only addition to the counter block: the counts per
+//      ray go to memory and the composite kernel sums them, 64 rays at a time (additions of thousands of workgroups to one
+//      line take 6.5 ns each: 12288 rays on three small planes, whole call: 232 us with
+//      valid and gathered samples added here too, 204 this way).
 // Four rays per workgroup: with eight the rays that see something crowd into fewer workgroups, with two or one the
 // samples of a round do not fill the waves (4096 rays of 128 samples on nine planes: 82 / 58 / 80 / 133 us with 8 / 4 / 2 /
 // 1 rays before the transmittance was spread over the lanes).
@@ -96,7 +99,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     lm_geom g, PlaneSet ps, int narrow, const float *__restrict__ den_w, const float *__restrict__ rays, uint32_t N, uint32_t row,
     int ent, int act, float shift, float distance_scale, float weight_thres, float term_eps, uint32_t cap_valid,
     uint32_t *__restrict__ app_first, uint32_t *__restrict__ app_cnt, uint32_t *__restrict__ app_idx, float *__restrict__ app_w,
-    uint32_t cap_app, float *__restrict__ acc_out, float *__restrict__ depth_out, uint32_t *__restrict__ counters) {
+    uint32_t cap_app, float *__restrict__ acc_out, float *__restrict__ depth_out, uint32_t *__restrict__ ray_valid,
+    uint32_t *__restrict__ ray_marched, uint32_t *__restrict__ counters) {
     __shared__ float s_ray[kRays][8];                 // origin, direction, ray parameter
     __shared__ uint64_t s_word[kRays][kWordsMax];     // decisions
     __shared__ uint16_t s_item[kRays][kRound];        // the round's samples
@@ -306,22 +310,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
 
     // ---- results and appearance entries: a contiguous range of slots per ray, in sample order
-    if (lane == 0) s_n[wave] = n_ray;
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t total = 0, done = 0, valid = 0;
+        uint32_t total = 0, over = 0;
         for (int i = 0; i < kRays; ++i) {
             s_first[i] = total;
             total += s_cnt[i];
-            done += s_done[i];
-            valid += s_n[i];
         }
-        // valid and appearance samples are neighbouring counters: one 64-bit addition (N S < 2^32: no carry)
-        static_assert(LM_STAT_N_VALID == 0 && LM_STAT_N_APP == 1, "counter order");
-        const unsigned long long add = ((unsigned long long)total << 32) | (limited ? 0u : valid);
-        uint32_t base = 0, over = 0;
-        if (add) base = (uint32_t)(atomicAdd(reinterpret_cast<unsigned long long *>(counters), add) >> 32);
-        if (done) atomicAdd(counters + LM_STAT_N_MARCHED, done);
+        const uint32_t base = total ? atomicAdd(counters + LM_STAT_N_APP, total) : 0u;
         for (int i = 0; i < kRays; ++i) {
             s_first[i] += base;
             // s_n: slots the ray may fill (0: no room, it keeps the background colour and is counted)
@@ -334,7 +330,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     __syncthreads();
     if (!have) return;
     const uint32_t first = s_first[wave], n = s_n[wave], cnt = s_cnt[wave], flat0 = r * (uint32_t)S;
-    if (lane == 0) { acc_out[r] = sum; app_first[r] = first; app_cnt[r] = n; }
+    if (lane == 0) { acc_out[r] = sum; app_first[r] = first; app_cnt[r] = n; ray_valid[r] = n_ray; ray_marched[r] = s_done[wave]; }
     if (lane == 1) depth_out[r] = sum;
     for (uint32_t j = lane; j < n; j += LM_WAVE) {
         app_idx[first + j] = flat0 + e_s[j];
@@ -354,11 +350,12 @@ bool lm_rays_kernel_takes(const lm_model *m, int64_t N) {
     return N <= LM_RAYS_LIMIT && m->geom.S <= 64 * kWordsMax && m->weight_thres * (float)(kEntriesMax - 2) >= 1.001f;
 }
 
-// Everything up to the appearance list for a small chunk; leaves the counters, acc, depth and the list behind like
-// lm_launch_cull_setup + lm_launch_march + lm_launch_app_slots.
+// Everything up to the appearance list for a small chunk; leaves acc, depth, the list and its counter behind like
+// lm_launch_cull_setup + lm_launch_march + lm_launch_app_slots, and per ray how many samples were valid and gathered, for
+// lm_launch_composite to sum.
 int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t row, uint32_t cap_valid, uint32_t *app_first,
                    uint32_t *app_cnt, uint32_t *app_idx, float *app_w, uint32_t cap_app, float *acc, float *depth,
-                   uint32_t *counters, hipStream_t st) {
+                   uint32_t *ray_valid, uint32_t *ray_marched, uint32_t *counters, hipStream_t st) {
     int dtype;
     if (int rc = lm_check_planes(m->density, m->n_planes, &dtype, nullptr)) return rc;
     LM_REQUIRE(m->act == LM_ACT_SOFTPLUS || m->act == LM_ACT_RELU, "unknown activation %d", m->act);
@@ -371,7 +368,8 @@ int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t ro
 #define LM_RAYS(T_)                                                                                                           \
     hipLaunchKernelGGL((k_rays<T_>), dim3((N + kRays - 1) / kRays), dim3(kBlock), lds, st, m->geom, ps, c_max <= Vec<T_>::V * kQuad ? 1 : 0, \
                        m->density_basis, rays, N, row, ent, m->act, m->density_shift, m->distance_scale, m->weight_thres,    \
-                       m->term_eps, cap_valid, app_first, app_cnt, app_idx, app_w, cap_app, acc, depth, counters)
+                       m->term_eps, cap_valid, app_first, app_cnt, app_idx, app_w, cap_app, acc, depth, ray_valid,       \
+                       ray_marched, counters)
     if (dtype == LM_F32) LM_RAYS(float);
     else if (c_max <= 16) LM_RAYS(Half4);
     else LM_RAYS(__half);

@@ -1,0 +1,56 @@
+"""What lm_render promises its callers holds for chunks that take the fused small-chunk kernels as it does for those that
+take the kernels per stage."""
+import ctypes as C
+
+import pytest
+import torch
+
+from landmark_amd import _lib as L
+from landmark_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _params(S=128, opt=1, thres=1e-3, gain=6.0, mask=True):
+    p = scenes.make_params(seed=7, gridSize=(14, 12, 10), near_far=[0.5, 4.5], n_importance=S, sampling_opt=opt, ndims=3,
+                           density_shift=0.0, step_ratio=12.0 / S)
+    for t in p.density_plane:
+        t.mul_(gain)
+    if mask:
+        p.alpha_volume = scenes.blob_occupancy((20, 18, 16), 8, 0.5, seed=3)
+        p.alpha_aabb = p.aabb.clone()
+    p.rayMarch_weight_thres = thres
+    return p
+
+
+def _model(p, **kw):
+    from landmark_amd.model import GridNeRFHIP
+
+    return GridNeRFHIP(p, device="cuda", mlp_precision="f16x2", **kw)
+
+
+def _rays():
+    return scenes.pinhole_rays(120, 110, 100.0, scenes.sphere_pose(2.5, 9)).cuda()  # 13200 rays: kernels per stage
+
+
+def _counts(t):
+    return [int(v) & 0xFFFFFFFF for v in t.cpu()]
+
+
+def test_counter_block_needs_the_alignment_of_its_words_only(gpu_lib):
+    """A counter block one word into a buffer (a caller's packed statistics): same counts, same picture, the words around
+    it untouched."""
+    m = _model(_params())
+    rays = _rays()[4000:7000]
+    buf = torch.full((L.LM_STAT_WORDS + 2,), 77, dtype=torch.int32, device="cuda")
+    odd = buf[1 : 1 + L.LM_STAT_WORDS]
+    assert odd.data_ptr() % 8 == 4
+    got = []
+    for cnt in (torch.zeros(L.LM_STAT_WORDS, dtype=torch.int32, device="cuda"), odd):
+        rgb, depth = torch.empty((3000, 3), device="cuda"), torch.empty(3000, device="cuda")
+        m.render_into(rays, rgb, depth, counters=cnt)
+        torch.cuda.synchronize()
+        got.append((rgb, depth, _counts(cnt)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
+    assert got[0][2][L.LM_STAT_N_APP] > 1000
+    assert int(buf[0]) == 77 and int(buf[-1]) == 77
