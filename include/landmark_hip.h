@@ -334,6 +334,14 @@ size_t lm_render_workspace_bytes(const lm_model *model, int64_t N);
 int lm_render(const lm_model *model, const float *rays, int64_t N, void *workspace, size_t workspace_bytes,
               float *rgb_map, float *depth_map, uint32_t *counters, void *stream);
 
+/* Which stages of an lm_render of N rays of this model are fused into one kernel: bits of LM_ROUTE_* (0: a kernel per
+ * stage), or a negative lm_status.  Results do not depend on it; it tells which stage times to expect. */
+enum {
+    LM_ROUTE_RAYS = 1, /* sampling up to the appearance list */
+    LM_ROUTE_SHADE = 2 /* appearance gather and colour network */
+};
+int lm_render_route(const lm_model *model, int64_t N);
+
 /* lm_render out of a workspace built into the library, for callers that cannot allocate device
  * memory or pass a workspace along: code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  No counterpart in the reference (its fused path allocates its buffers

@@ -21,6 +21,7 @@ LM_F32, LM_F16, LM_U8, LM_CELLS = 0, 1, 2, 3
 LM_SAMPLER_AABB, LM_SAMPLER_HULL = 0, 1
 LM_ACT_SOFTPLUS, LM_ACT_RELU = 0, 1
 LM_MLP_F32, LM_MLP_F16, LM_MLP_BF16, LM_MLP_F16X2 = 0, 1, 2, 3
+LM_ROUTE_RAYS, LM_ROUTE_SHADE = 1, 2
 MLP_PREC = {"f32": LM_MLP_F32, "fp32": LM_MLP_F32, "f16": LM_MLP_F16, "fp16": LM_MLP_F16, "bf16": LM_MLP_BF16, "f16x2": LM_MLP_F16X2}
 
 
@@ -83,6 +84,7 @@ SYMBOLS = {
     "lm_composite_rgb": (C.c_int, [_I64, _P, _P, _P, _P, _P, _I32, _P, _P]),
     "lm_render_workspace_bytes": (_SZ, [C.POINTER(LmModel), _I64]),
     "lm_app_features": (C.c_int, [C.POINTER(LmModel), _P, _P, _P, _P, _P]),
+    "lm_render_route": (C.c_int, [C.POINTER(LmModel), _I64]),
     "lm_render": (C.c_int, [C.POINTER(LmModel), _P, _I64, _P, _SZ, _P, _P, _P, _P]),
     "lm_render_static": (C.c_int, [C.POINTER(LmModel), _P, _I64, _P, _P, _P, _P]),
     "lm_generate_rays": (C.c_int, [_P, _P, _P, _I32, _I32, _P, _P]),

@@ -223,6 +223,14 @@ extern "C" size_t lm_render_workspace_bytes(const lm_model *m, int64_t N) {
     return carve(nullptr, N, m->geom.S, K, !lm_app_feat_supported(m), m->weight_thres, m->cap_valid, m->cap_app).total;
 }
 
+extern "C" int lm_render_route(const lm_model *m, int64_t N) {
+    int K;
+    if (int rc = check_model(m, &K)) return rc;
+    LM_REQUIRE(N >= 0, "negative ray count");
+    if (!lm_rays_kernel_takes(m, N)) return 0;
+    return LM_ROUTE_RAYS | (lm_shade_takes(m, N, K) ? LM_ROUTE_SHADE : 0);
+}
+
 extern "C" int lm_render(const lm_model *m, const float *rays, int64_t N, void *workspace, size_t workspace_bytes,
                          float *rgb_map, float *depth_map, uint32_t *counters, void *stream) {
     int K;

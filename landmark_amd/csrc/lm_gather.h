@@ -7,6 +7,11 @@
 
 #include "lm_common.h"
 
+// chunks of up to this many rays are small: a kernel from rays to appearance entries (lm_ray.hip), or a wave per ray
+#ifndef LM_RAYS_LIMIT
+#define LM_RAYS_LIMIT 12288
+#endif
+
 namespace {
 
 constexpr int kBlock = 256;

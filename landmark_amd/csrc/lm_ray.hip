@@ -30,16 +30,11 @@
 #include "lm_cull.h"
 #include "lm_gather.h"
 
-// chunks of up to this many rays
-#ifndef LM_RAYS_LIMIT
-#define LM_RAYS_LIMIT 12288
-#endif
-
 namespace {
 
 constexpr int kRays = kBlock / LM_WAVE;  // rays per workgroup: a wave owns one
 constexpr int kWordsMax = 64;            // a ray's decisions: up to 64 words of 64 samples
-constexpr int kEntriesMax = 1024;        // appearance entries of a ray: at most 1 / weight threshold and S
+constexpr int kEntriesMax = 1024;        // appearance entries of a ray: at most S and 1 / weight threshold
 constexpr int kRound = 64;               // samples a ray contributes to a round
 
 // density_sum_n with G planes' loads in flight; planes of one channel group per lane only (G > 1)
@@ -345,9 +340,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 
 int lm_check_planes(const lm_plane *planes, int32_t n, int *dtype_out, int *K_out);
 
-// Chunks of up to LM_RAYS_LIMIT rays whose decisions fit 64 words per ray and whose appearance entries fit LDS
+// Chunks of up to LM_RAYS_LIMIT rays whose decisions fit 64 words per ray and whose appearance entries fit LDS: one per
+// sample, or as many as weights above the threshold can be (they sum to at most 1).
 bool lm_rays_kernel_takes(const lm_model *m, int64_t N) {
-    return N <= LM_RAYS_LIMIT && m->geom.S <= 64 * kWordsMax && m->weight_thres * (float)(kEntriesMax - 2) >= 1.001f;
+    const bool entries_fit = m->geom.S <= kEntriesMax || m->weight_thres * (float)(kEntriesMax - 2) >= 1.001f;
+    return N <= LM_RAYS_LIMIT && m->geom.S <= 64 * kWordsMax && entries_fit;
 }
 
 // Everything up to the appearance list for a small chunk; leaves acc, depth, the list and its counter behind like

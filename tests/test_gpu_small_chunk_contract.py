@@ -54,3 +54,26 @@ def test_counter_block_needs_the_alignment_of_its_words_only(gpu_lib):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
     assert got[0][2][L.LM_STAT_N_APP] > 1000
     assert int(buf[0]) == 77 and int(buf[-1]) == 77
+
+
+@pytest.mark.parametrize("S,opt,thres,route", [(128, 1, 1e-4, L.LM_ROUTE_RAYS), (128, 1, 0.0, L.LM_ROUTE_RAYS), (1024, 0, 1e-4, L.LM_ROUTE_RAYS),
+                                               (1025, 0, 1e-4, 0), (1300, 0, 0.0, 0), (5000, 0, 1e-3, 0)])
+@pytest.mark.parametrize("term", [0.0, 1e-3])
+def test_low_thresholds_and_long_rays_in_small_chunks(gpu_lib, S, opt, thres, route, term):
+    """Thresholds that let a ray have an entry per sample, and rays the fused kernel does not hold: the same picture and counts as
+    the kernels for large chunks give."""
+    m = _model(_params(S, opt, thres), term_eps=term)
+    rays = _rays()
+    whole, _ = m(rays, N_samples=S, chunk=rays.shape[0])
+    total = _counts(m.counters)
+    n_valid = n_app = at = 0
+    for n in (1, 7, 500, 12288, 404):
+        st = m._model_struct(S, True)
+        assert gpu_lib.lm_render_route(C.byref(st), n) & L.LM_ROUTE_RAYS == route
+        part, _ = m(rays[at : at + n], N_samples=S, chunk=n)
+        c = _counts(m.counters)
+        assert c[L.LM_STAT_OVERFLOW] == 0
+        n_valid, n_app = n_valid + c[L.LM_STAT_N_VALID], n_app + c[L.LM_STAT_N_APP]
+        assert torch.equal(part["rgb_map"], whole["rgb_map"][at : at + n]) and torch.equal(part["depth_map"], whole["depth_map"][at : at + n])
+        at += n
+    assert at == rays.shape[0] and n_valid == total[L.LM_STAT_N_VALID] and n_app == total[L.LM_STAT_N_APP] > 1000
