@@ -430,8 +430,14 @@ static bool shade_covers(const lm_model *m, int K) { return lm_app_feat_supporte
 // there, 217 - 225 here; 3.6 million of the production shape 337 and 337; 7.3 million 555 and 567).  The fp32 network's
 // matrix steps take eight times as long, its line lies at half a million (4096 rays of 128 samples, 46 000 entries:
 // 145 and 119 us; 8192 rays: 203 and 218).
+// With a threshold far below the weights of a uniform fog (1 / S) nearly every valid sample is an entry, three to six times
+// as many: the lines lie at a third (threshold 0, three small planes, here / there: 2048 rays of 128 samples 146 / 155 us,
+// 4096 258 / 226, 12288 685 / 527; nine planes 8192 rays 344 / 348, 12288 483 / 455; fp32 network 1024 rays 139 / 155,
+// 4096 443 / 363).
 bool lm_shade_takes(const lm_model *m, int64_t N, int K) {
-    return shade_covers(m, K) && N * m->geom.S <= (m->mlp_prec == LM_MLP_F32 ? 1ll << 19 : 3ll << 20);
+    const int64_t limit = m->mlp_prec == LM_MLP_F32 ? 1ll << 19 : 3ll << 20;
+    const bool most_samples = m->weight_thres * (float)m->geom.S < 1e-2f;
+    return shade_covers(m, K) && N * m->geom.S <= (most_samples ? limit / 3 : limit);
 }
 
 // compute_appfeature at given points: up to here a tile per workgroup beats k_app_feat's tile per wave.  Nine planes, split

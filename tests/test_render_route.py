@@ -52,6 +52,14 @@ def test_shading_in_one_kernel_up_to_a_number_of_candidate_samples(lib, prec, S,
     assert lib.lm_render_route(C.byref(_host_model(S, 1e-3, app_channels=40, prec=prec)), n) == L.LM_ROUTE_RAYS
 
 
+@pytest.mark.parametrize("prec,thres,n,fused", [(L.LM_MLP_F16X2, 0.0, 8192, True), (L.LM_MLP_F16X2, 0.0, 8193, False), (L.LM_MLP_F16X2, 7e-5, 8193, False),
+                                                (L.LM_MLP_F16X2, 1e-4, 8193, True), (L.LM_MLP_F16X2, -1.0, 8193, False), (L.LM_MLP_F32, 0.0, 1365, True),
+                                                (L.LM_MLP_F32, 0.0, 1366, False), (L.LM_MLP_F32, 1e-4, 1366, True)])
+def test_shading_limit_where_nearly_every_valid_sample_is_an_entry(lib, prec, thres, n, fused):
+    got = lib.lm_render_route(C.byref(_host_model(128, thres, prec=prec)), n)
+    assert got == L.LM_ROUTE_RAYS | (L.LM_ROUTE_SHADE if fused else 0)
+
+
 def test_bad_arguments_are_refused(lib):
     assert lib.lm_render_route(None, 4) < 0
     assert lib.lm_render_route(C.byref(_host_model(0, 1e-3)), 4) < 0
