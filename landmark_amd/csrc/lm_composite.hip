@@ -131,10 +131,10 @@ __global__ __launch_bounds__(kBlock) void k_composite(uint64_t N, const uint32_t
                                                            uint32_t row, float *__restrict__ rgb_map, RayStats stats) {
     const uint64_t o = (uint64_t)blockIdx.x * (kBlock / 4) + threadIdx.x / 4;
     const unsigned ch = threadIdx.x & 3u;
-    __shared__ uint32_t s_sum[2];
+    __shared__ uint32_t s_sum[2 + LM_RAY_BINS];  // samples valid and gathered, rays by their number of valid samples
     uint32_t n_valid = 0, n_marched = 0;
     if constexpr (STATS) {
-        if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+        if (threadIdx.x < 2 + LM_RAY_BINS) s_sum[threadIdx.x] = 0;
         if (o < N && ch == 3u) { n_valid = stats.valid[o]; n_marched = stats.marched[o]; }
     }
     if (o < N && ch != 3u) {
@@ -162,11 +162,15 @@ __global__ __launch_bounds__(kBlock) void k_composite(uint64_t N, const uint32_t
     }
     if constexpr (STATS) {
         __syncthreads();
-        if (n_valid) atomicAdd(&s_sum[0], n_valid);
+        if (n_valid) {
+            atomicAdd(&s_sum[0], n_valid);
+            atomicAdd(&s_sum[2 + lm_ray_bin(n_valid)], 1u);
+        }
         if (n_marched) atomicAdd(&s_sum[1], n_marched);
         __syncthreads();
-        if (threadIdx.x == 0 && stats.count_valid && s_sum[0]) atomicAdd(stats.counters + LM_STAT_N_VALID, s_sum[0]);
-        if (threadIdx.x == 1 && s_sum[1]) atomicAdd(stats.counters + LM_STAT_N_MARCHED, s_sum[1]);
+        const unsigned t = threadIdx.x;
+        if (t < 2 + LM_RAY_BINS && s_sum[t] && (t != 0u || stats.count_valid))
+            atomicAdd(stats.counters + (t == 0u ? LM_STAT_N_VALID : t == 1u ? LM_STAT_N_MARCHED : LM_STAT_BINS + t - 2u), s_sum[t]);
     }
 }
 

@@ -77,3 +77,19 @@ def test_low_thresholds_and_long_rays_in_small_chunks(gpu_lib, S, opt, thres, ro
         assert torch.equal(part["rgb_map"], whole["rgb_map"][at : at + n]) and torch.equal(part["depth_map"], whole["depth_map"][at : at + n])
         at += n
     assert at == rays.shape[0] and n_valid == total[L.LM_STAT_N_VALID] and n_app == total[L.LM_STAT_N_APP] > 1000
+
+
+@pytest.mark.parametrize("S,opt", [(128, 1), (300, 0), (20, 1)])
+def test_rays_by_their_number_of_valid_samples_are_counted(gpu_lib, S, opt):
+    """LM_STAT_BINS .. BINS + 3: the same rays per bin, whether a chunk takes the fused kernel or the kernels per stage."""
+    m = _model(_params(S, opt))
+    rays = _rays()
+    cull = m.sample_cull(rays, N_samples=S)
+    n = cull["ray_valid"].sum(1)
+    assert int(n.max()) >= (64 if S > 64 else 12)
+    for at, size in ((0, 13200), (1000, 12200), (5000, 3001), (6000, 5)):
+        c = n[at : at + size]
+        want = [int(v) for v in ((c >= 64).sum(), ((c >= 32) & (c < 64)).sum(), ((c >= 12) & (c < 32)).sum(), ((c > 0) & (c < 12)).sum())]
+        m(rays[at : at + size], N_samples=S, chunk=size)
+        got = _counts(m.counters)
+        assert got[L.LM_STAT_BINS : L.LM_STAT_BINS + 4] == want and got[L.LM_STAT_N_VALID] == int(c.sum())
