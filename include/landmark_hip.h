@@ -36,8 +36,8 @@ extern "C" {
 #endif
 
 /* Changes whenever a struct, an enum value or the meaning of an argument does (2: 16-word counter block;
- * 3: workspace capacities in lm_model, LM_STAT_OVERFLOW). */
-#define LM_ABI_VERSION 4
+ * 3: workspace capacities in lm_model, LM_STAT_OVERFLOW; 4: lm_geom.vol_coarse; 5: lm_model.skip_lost, fused stages). */
+#define LM_ABI_VERSION 5
 #define LM_MAX_PLANES 12 /* ndims * len(resMode) */
 
 typedef enum lm_status {
@@ -143,16 +143,18 @@ typedef struct lm_model {
     int32_t mlp_prec;   /* LM_MLP_* the packed weights were packed for */
     const void *mlp_packed; /* device copy of the buffer written by lm_mlp_pack */
     int32_t white_bg;
-    float term_eps; /* > 0: stop marching a ray once transmittance < term_eps.  0: gather every valid sample.  < 0: stop
-                     * where no later sample can change opacity, depth or the appearance list, same bits as 0; the caller
-                     * promises finite tables (a NaN behind that point would not be seen) and a positive distance_scale */
+    float term_eps; /* > 0: stop marching a ray once transmittance < term_eps.  Otherwise: gather every valid sample */
     /* Hint: the chunk's rays are the pixels of an image stored row by row, ray_row of them per
      * row (the chunk may start anywhere in a row).  lm_render then visits rays in 8 x 8 pixel
      * tiles, so that rays handled together are neighbours in both directions and share more of
      * the tables' cache lines.  Results and their order do not depend on it.  0 or not a
      * multiple of 8: rays are visited in the order given. */
     int32_t ray_row;
-    int32_t reserved_;
+    /* Not 0, with term_eps not above 0: a ray stops where no later sample can change a bit of its opacity, its depth or its
+     * appearance list (rays of small chunks that march a wave each keep every sample).  The caller promises densities
+     * finite everywhere (a NaN behind that point would not be seen), a positive distance_scale, and depth tables that
+     * ascend in even steps, as both samplers' do.  0: no promise. */
+    int32_t skip_lost;
     /* Workspace capacities of one lm_render call, in samples: room for the chunk's valid samples and for its
      * appearance samples (weight > weight_thres).  0 = the worst case (every sample valid, every ray with
      * min(S, 1 / weight_thres) appearance samples), which cannot overflow; the reference's fused path sizes its
@@ -173,7 +175,7 @@ typedef struct lm_model {
 } lm_model;
 
 /* Counters written by lm_render (device memory, LM_STAT_WORDS x uint32). */
-/* N_MARCHED: valid samples whose density was gathered (< N_VALID with early termination);
+/* N_MARCHED: valid samples whose density was gathered (< N_VALID with early termination or skip_lost);
  * BINS..BINS+3: rays with valid samples, by how many they have (>= 64, >= 32, >= 12, fewer): the
  * marching queue hands out the long rays first; QUEUE..QUEUE+7: internal cursors of that queue,
  * one per XCD.  Two lm_render calls that may run at the same time (different streams) need a

@@ -392,11 +392,13 @@ struct BitWalk {
     }
 };
 
-// term_eps < 0: true when nothing behind the present sample can change what the ray leaves behind, not even in the last
-// bit.  Later weights are at most the transmittance (alpha lies in 0 .. 1, the factors do not exceed 1, depths ascend to
+// lm_model.skip_lost: true when nothing behind the present sample can change what the ray leaves behind, not even in the
+// last bit.  Later weights are at most the transmittance (alpha lies in 0 .. 1, the factors do not exceed 1, depths ascend to
 // z_last): below 2^-26 of the opacity they are under half a unit in its last place (above 2^-25 of its value), and so is
 // weight x depth against the depth sum, and none of them passes the appearance threshold.  `dist` > 0 by a margin: the
-// ray's depths do ascend, roundings included.  Needs finite densities (the caller's promise, see landmark_hip.h).
+// ray's depths do ascend, roundings included.  Needs finite densities (the caller's promise).
 __device__ __forceinline__ bool lm_rest_is_lost(float Tr, float acc, float depth, float dist, float z_last, float weight_thres) {
     return Tr <= weight_thres && Tr < acc * 0x1p-26f && Tr * z_last < depth * 0x1p-26f && dist > 1e-6f * z_last;
 }
+// What the marching kernels are given: a threshold above 0, -1 for "stop where the rest is lost", or 0 for "never stop"
+inline float lm_stop_value(const lm_model &m) { return m.term_eps > 0.0f ? m.term_eps : m.skip_lost ? -1.0f : 0.0f; }

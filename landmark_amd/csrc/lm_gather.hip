@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kBlock) void k_app_list(lm_geom g, PlaneSet ps, int
 // stay busy whatever the rays' lengths.  Two things follow from walking rays in lock step:
 // neighbouring rays are at similar depths in the same load instruction, so their corner
 // texels share cache lines; and a ray can stop once its transmittance is below term_eps,
-// before the density of the samples behind is ever fetched, or (term_eps < 0) once nothing behind can change its results
+// before the density of the samples behind is ever fetched, or (skip_lost) once nothing behind can change its results
 // (155.8 -> 135 million samples gathered for 518400 rays of 3544 steps, 8.4 -> 6.2 million for 160000 rays of 128).  With term_eps = 0 the weights
 // are those of the separate density + weights kernels, bit for bit (same operations, and the
 // transmittance is the same sequential product torch.cumprod forms, app/tools/utils.py:51-64).
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
                                                   const uint32_t *__restrict__ bins, uint32_t n_rays,
                                                   uint32_t *__restrict__ queue,
                                                   int act, float shift, float distance_scale, float weight_thres,
-                                                  float term_eps, float *__restrict__ w_valid,
+                                                  float stop, float *__restrict__ w_valid,
                                                   float *__restrict__ acc_out, float *__restrict__ depth_out,
                                                   uint32_t *__restrict__ app_cnt, uint32_t *__restrict__ p_end_out,
                                                   uint32_t *__restrict__ n_marched) {
@@ -263,10 +263,10 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
                     depth += wgt * z_n[n];
                     cnt += wgt > weight_thres;
                     ++p;
-                    finish = term_eps > 0.0f && Tr < term_eps;
+                    finish = stop > 0.0f && Tr < stop;
                 }
                 if (n_have < NS) finish = true;  // the ray's last samples
-                else if (term_eps < 0.0f && !finish)
+                else if (stop < 0.0f && !finish)
                     finish = lm_rest_is_lost(Tr, acc, depth, quad_lane(dist, NS - 1), z_last, weight_thres);
             }
             if (finish) {
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
 // memory round trip.  The transmittance then runs through the word's valid samples in order, every lane
 // computing the same scalars from values read off the owning lanes: the same operations in the same order as
 // the quad march, hence the same bits (weights, sums, counts, the sample at which a ray stops), whichever of
-// the two kernels a chunk's size selects.  It does not stop at lost samples (term_eps < 0 is 0 here).
+// the two kernels a chunk's size selects.  It does not stop at lost samples.
 // Whole calls, quad per ray / wave per ray: 4096 rays of 4726 samples 3570 / 1510 us, 4096 rays of 7088 5000 / 1990,
 // 1024 rays of 7088 2430 / 950, 12288 rays of 7088 5700 / 3750, 4096 rays of 3544 at threshold 1e-4 2950 / 1790.
 template <typename T>
@@ -896,7 +896,7 @@ int lm_launch_march(const lm_model *m, const float *rays, const uint64_t *bitmap
     hipLaunchKernelGGL((k_march<T_, NS_>), dim3(resident_grid(reinterpret_cast<const void *>(&k_march<T_, NS_>))),         \
                        dim3(kBlock), 0, st, m->geom, ps, m->density_basis, rays, bitmap,   \
                        p_first, word_mask, ray_list, bins, n_rays, queue, m->act, m->density_shift, m->distance_scale,            \
-                       m->weight_thres, m->term_eps, w_valid, acc, depth, app_cnt, p_end, n_marched)
+                       m->weight_thres, lm_stop_value(*m), w_valid, acc, depth, app_cnt, p_end, n_marched)
     // Four samples per round: one per lane of the quad for the footprint arithmetic, 24 loads per lane and plane
     // in flight, half as many dependent round trips per ray as with two (1080p frame, nine fp32 planes: 2.70 ->
     // 2.50 ms although the kernel then holds 223 registers and two waves per SIMD instead of three).

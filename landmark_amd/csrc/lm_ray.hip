@@ -21,7 +21,7 @@
 // samples of a round do not fill the waves (4096 rays of 128 samples on nine planes: 82 / 58 / 80 / 133 us with 8 / 4 / 2 /
 // 1 rays before the transmittance was spread over the lanes).
 // Measured against zeroed bitmap + cull + march with a wave per ray + list: 4096 rays as above 93 -> 45 us, 8192 rays of
-// 886 samples on three planes 393 -> 310 us, 1024 rays on three 256^2 planes 51 -> 23 us.  With term_eps < 0 (rays
+// 886 samples on three planes 393 -> 310 us, 1024 rays on three 256^2 planes 51 -> 23 us.  With skip_lost (rays
 // stop after the round behind which nothing can change their results) the second takes 229 us, the third 20.
 // Operations and order per ray are those of the kernels for large chunks, hence the same bits.
 #include <algorithm>
@@ -92,7 +92,7 @@ __device__ __forceinline__ void density_sum_planes(const PlaneSet &ps, const flo
 template <typename T>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_rays(
     lm_geom g, PlaneSet ps, int narrow, const float *__restrict__ den_w, const float *__restrict__ rays, uint32_t N, uint32_t row,
-    int ent, int act, float shift, float distance_scale, float weight_thres, float term_eps, uint32_t cap_valid,
+    int ent, int act, float shift, float distance_scale, float weight_thres, float stop, uint32_t cap_valid,
     uint32_t *__restrict__ app_first, uint32_t *__restrict__ app_cnt, uint32_t *__restrict__ app_idx, float *__restrict__ app_w,
     uint32_t cap_app, float *__restrict__ acc_out, float *__restrict__ depth_out, uint32_t *__restrict__ ray_valid,
     uint32_t *__restrict__ ray_marched, uint32_t *__restrict__ counters) {
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             }
             lm_wave_lds_fence();
             float w_m = a_m * s_val[wave][lane];
-            const uint64_t over = __ballot(mine && term_eps > 0.0f && s_val[wave][lane + 1] < term_eps);
+            const uint64_t over = __ballot(mine && stop > 0.0f && s_val[wave][lane + 1] < stop);
             if (over) used = (uint32_t)__ffsll((unsigned long long)over);
             w_m = lane < used ? w_m : 0.0f;
             s_val[wave][lane] = w_m;
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 }
             }
             if (over) left = 0u;
-            else if (term_eps < 0.0f && left) {
+            else if (stop < 0.0f && left) {
                 auto of = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
                 const float z_last = lm_sample_z(g, s_ray[wave][6], S - 1), dist = z_last - of(z_m, 0);
                 if (lm_rest_is_lost(of(Tr, 0), of(sum, 0), of(sum, 1), dist / (float)S, z_last, weight_thres)) left = 0u;
@@ -365,7 +365,7 @@ int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t ro
 #define LM_RAYS(T_)                                                                                                           \
     hipLaunchKernelGGL((k_rays<T_>), dim3((N + kRays - 1) / kRays), dim3(kBlock), lds, st, m->geom, ps, c_max <= Vec<T_>::V * kQuad ? 1 : 0, \
                        m->density_basis, rays, N, row, ent, m->act, m->density_shift, m->distance_scale, m->weight_thres,    \
-                       m->term_eps, cap_valid, app_first, app_cnt, app_idx, app_w, cap_app, acc, depth, ray_valid,       \
+                       lm_stop_value(*m), cap_valid, app_first, app_cnt, app_idx, app_w, cap_app, acc, depth, ray_valid,       \
                        ray_marched, counters)
     if (dtype == LM_F32) LM_RAYS(float);
     else if (c_max <= 16) LM_RAYS(Half4);

@@ -114,7 +114,7 @@ class GridNeRFHIP:
             self._den_w = params.basis_den.detach().to(self.device, torch.float32).reshape(-1).contiguous()
             if self._den_w.numel() != sum(pl.C for pl in self._density):
                 raise L.LandmarkError("basis_den width does not match the density planes")
-        # rays may stop where the rest cannot change their results (lm_model.term_eps < 0) if the densities are finite
+        # rays may stop where the rest cannot change their results (lm_model.skip_lost) if the densities are finite
         self._finite_densities = self._density_bound(torch.stack(peaks).cpu().numpy()) < 1e30 and 0.0 < float(params.distance_scale) < 1e30
         # --- colour network; with encode_app the 48 latent columns of the first layer fold into its bias
         self.encode_app = bool(params.encode_app)
@@ -406,8 +406,9 @@ class GridNeRFHIP:
         prec, packed = self._pack_mlp(self.mlp_precision)
         m.mlp_prec, m.mlp_packed = prec, packed.data_ptr()
         m.white_bg = int(bool(white_bg))
+        m.term_eps = self.term_eps
         # exact results asked for: a ray may still stop once nothing behind can change them (finite densities only)
-        m.term_eps = self.term_eps if self.term_eps > 0 else (-1.0 if self._finite_densities else 0.0)
+        m.skip_lost = int(self._finite_densities)
         m.ray_row = int(self.ray_row_length)
         return m
 

@@ -93,3 +93,26 @@ def test_rays_by_their_number_of_valid_samples_are_counted(gpu_lib, S, opt):
         m(rays[at : at + size], N_samples=S, chunk=size)
         got = _counts(m.counters)
         assert got[L.LM_STAT_BINS : L.LM_STAT_BINS + 4] == want and got[L.LM_STAT_N_VALID] == int(c.sum())
+
+
+@pytest.mark.parametrize("n", [3000, 13200])
+def test_a_negative_termination_value_promises_nothing(gpu_lib, n):
+    """term_eps below zero is no termination, as zero is; stopping at lost samples is asked for by skip_lost alone."""
+    S = 300
+    m = _model(_params(S, 0, gain=60.0, mask=False))
+    rays = _rays()[:n]
+    ws = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
+    marched = {}
+    for term, skip in ((0.0, 0), (-1.0, 0), (-1.0, 1), (0.0, 1)):
+        st = m._build_model_struct(S, True)
+        st.term_eps, st.skip_lost = term, skip
+        cnt = torch.zeros(L.LM_STAT_WORDS, dtype=torch.int32, device="cuda")
+        rgb, depth = torch.empty((n, 3), device="cuda"), torch.empty(n, device="cuda")
+        assert gpu_lib.lm_render_workspace_bytes(C.byref(st), n) <= ws.numel()
+        L.check(gpu_lib.lm_render(C.byref(st), rays.data_ptr(), n, ws.data_ptr(), ws.numel(), rgb.data_ptr(), depth.data_ptr(), cnt.data_ptr(),
+                                  L.current_stream()), "lm_render")
+        torch.cuda.synchronize()
+        c = _counts(cnt)
+        marched[term, skip] = c[L.LM_STAT_N_VALID] - c[L.LM_STAT_N_MARCHED]
+    assert marched[0.0, 0] == 0 and marched[-1.0, 0] == 0
+    assert marched[0.0, 1] == marched[-1.0, 1] > 0
