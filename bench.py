@@ -19,6 +19,7 @@ network never runs; `--density-shift -10` reproduces that case).
 from __future__ import annotations
 
 import argparse
+import ctypes as C
 import json
 import os
 import sys
@@ -63,6 +64,18 @@ def log(*a):
 
 def plane_bytes_per_sample(planes):
     return sum(4 * pl.C * (4 if pl.dtype == 0 else 2) for pl in planes)
+
+
+def stage_kernels(route):
+    """Where a frame's time is, as (stage name, indices of lm_render's stage intervals, kernel), dominant candidates only.
+    `route`: LM_ROUTE_* bits of its whole chunks.  Small chunks have fused kernels: everything up to the appearance
+    list then falls into the first interval and the next two are empty, and appearance gather and colour network share
+    the fourth with the fifth empty, so no figure can be given for the parts."""
+    from landmark_amd import _lib as L
+
+    front = [("cull", (0, 1, 2), "k_rays")] if route & L.LM_ROUTE_RAYS else [("density_march", (1,), "k_march")]
+    back = [("app_gather", (3, 4), "k_shade")] if route & L.LM_ROUTE_SHADE else [("app_gather", (3,), "k_app_feat"), ("colour", (4,), "k_mlp")]
+    return front + back
 
 
 # ----------------------------------------------------------------------------------------
@@ -247,39 +260,49 @@ def bench_frame(args, workload):
     stages = {}
     for i, nm in enumerate(L.STAGE_NAMES):
         stages[nm] = {"ms_per_frame": round(stage_ms[i], 4)}
+    # (a last chunk small enough for the fused kernels while the others are not moves its share of the time between stages)
+    n = min(chunk, N)
+    route = model.lib.lm_render_route(C.byref(model._model_struct(S, True, model.capacities(n, S))), n)
+    groups = {nm: (sum(stage_ms[i] for i in at), kernel) for nm, at, kernel in stage_kernels(route)}
     # GB/s figures of the gathers are in gather-convention bytes: every corner load of every sample, no reuse
-    stages["density_march"].update(bytes_per_sample=dens_B, samples=n_marched,
-                                   convention_GBps=round(n_marched * dens_B / max(stage_ms[1], 1e-9) / 1e6, 1))
-    stages["app_gather"].update(bytes_per_sample=app_B, samples=n_app,
-                                convention_GBps=round(n_app * app_B / max(stage_ms[3], 1e-9) / 1e6, 1),
-                                basis_TFLOPs=round(n_app * basis_flop / max(stage_ms[3], 1e-9) / 1e9, 2))
-    stages["colour"].update(rows=n_app, TFLOPs=round(n_app * MLP_FLOP_PER_ROW / max(stage_ms[4], 1e-9) / 1e9, 2),
-                            frac_of_mfma_peak=round(n_app * MLP_FLOP_PER_ROW / max(stage_ms[4], 1e-9) / 1e9 / MFMA_PEAK_TFLOPS[args.mlp], 4))
-    # occupancy lookups: 1 byte per sample from the cell table (8 x 4 bytes with a float volume), upper bound
-    # every sample; 1 bit per sample and 24 bytes per ray besides
-    cull_B = (1 if model._vol_dtype == L.LM_CELLS else 32 if model._vol is not None else 0) + 0.125
-    stages["cull"].update(bytes_per_sample=cull_B, Gsamples_per_s=round(N * S / (stage_ms[0] * 1e-3) / 1e9, 1),
-                          GBps=round((N * S * cull_B + N * 24) / (stage_ms[0] * 1e-3) / 1e9, 1))
+    if route & L.LM_ROUTE_RAYS:
+        stages["cull"]["kernel"] = "k_rays: cull, density march and appearance list of small chunks"
+    else:
+        stages["density_march"].update(bytes_per_sample=dens_B, samples=n_marched,
+                                       convention_GBps=round(n_marched * dens_B / max(stage_ms[1], 1e-9) / 1e6, 1))
+        # occupancy lookups: 1 byte per sample from the cell table (8 x 4 bytes with a float volume), upper bound
+        # every sample; 1 bit per sample and 24 bytes per ray besides
+        cull_B = (1 if model._vol_dtype == L.LM_CELLS else 32 if model._vol is not None else 0) + 0.125
+        stages["cull"].update(bytes_per_sample=cull_B, Gsamples_per_s=round(N * S / (stage_ms[0] * 1e-3) / 1e9, 1),
+                              GBps=round((N * S * cull_B + N * 24) / (stage_ms[0] * 1e-3) / 1e9, 1))
+        stages["app_list"].update(GBps=round((n_marched * 4 + N * S / 8 + n_app * 8 + N * 16) / (stage_ms[2] * 1e-3) / 1e9, 1))
+    if route & L.LM_ROUTE_SHADE:
+        stages["app_gather"]["kernel"] = "k_shade: appearance gather and colour network of small chunks"
+    else:
+        stages["app_gather"].update(bytes_per_sample=app_B, samples=n_app,
+                                    convention_GBps=round(n_app * app_B / max(stage_ms[3], 1e-9) / 1e6, 1),
+                                    basis_TFLOPs=round(n_app * basis_flop / max(stage_ms[3], 1e-9) / 1e9, 2))
+        stages["colour"].update(rows=n_app, TFLOPs=round(n_app * MLP_FLOP_PER_ROW / max(stage_ms[4], 1e-9) / 1e9, 2),
+                                frac_of_mfma_peak=round(n_app * MLP_FLOP_PER_ROW / max(stage_ms[4], 1e-9) / 1e9 / MFMA_PEAK_TFLOPS[args.mlp], 4))
     stages["composite"].update(GBps=round((n_app * 16 + N * 32) / max(stage_ms[5], 1e-9) / 1e6, 1))  # w + rgb per slot; first, count, acc in and rgb out per ray
-    stages["app_list"].update(GBps=round((n_marched * 4 + N * S / 8 + n_app * 8 + N * 16) / (stage_ms[2] * 1e-3) / 1e9, 1))
 
     # dominant kernel -> roofline object
-    cand = {"density_march": stage_ms[1], "app_gather": stage_ms[3], "colour": stage_ms[4]}
-    dom = max(cand, key=cand.get)
-    avg_ms = cand[dom] / launches
-    if dom == "colour":
+    dom = max(groups, key=lambda nm: groups[nm][0])
+    dom_ms, kernel = groups[dom]
+    avg_ms = dom_ms / launches
+    if kernel == "k_mlp":
         ach = stages["colour"]["TFLOPs"]
         peak = MFMA_PEAK_TFLOPS[args.mlp]
         roof = {"kernel": "k_mlp", "bound": "mfma", "achieved": ach, "peak": peak, "unit": "TFLOP/s",
                 "frac": round(ach / peak, 4), "traffic": None}
     else:
-        kernel = "k_march" if dom == "density_march" else "k_app_feat"
-        conv = stages[dom]["convention_GBps"]
+        samples, per_sample = (n_marched, dens_B) if kernel in ("k_march", "k_rays") else (n_app, app_B)
+        conv = round(samples * per_sample / max(dom_ms, 1e-9) / 1e6, 1)
         found = measured_traffic(name, chunk, args.mlp, "auto" if term_auto else f"{term_eps:g}", kernel) \
             if int(model.ray_row_length) == W else None
         roof = {"kernel": kernel, "bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "convention": "gather, no reuse: every corner load of every sample counted, line tables excluded",
-                "convention_bytes_per_launch": round(stages[dom]["samples"] * stages[dom]["bytes_per_sample"] / launches),
+                "convention_bytes_per_launch": round(samples * per_sample / launches),
                 "convention_GBps": conv}
         if found:
             # bytes the launch moved past the L2 (rocprofv3 counters, summarised under profiles/) / its duration here

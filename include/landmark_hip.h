@@ -116,7 +116,9 @@ typedef struct lm_geom {
     const uint8_t *vol_coarse;
 } lm_geom;
 
-/* stages of lm_render, in launch order */
+/* stages of lm_render, in launch order.  Small chunks have fused kernels (lm_render_route): with LM_ROUTE_RAYS the time from
+ * sampling to the appearance list falls into stage CULL and DENSITY and WEIGHTS take none, with LM_ROUTE_SHADE the
+ * colour network's falls into APP and COLOUR takes none. */
 enum {
     LM_STAGE_CULL = 1,      /* sampling + culling + compaction, list of rays with valid samples */
     LM_STAGE_DENSITY = 2,   /* density gather fused with the per-ray transmittance march */
