@@ -21,7 +21,8 @@ __device__ __forceinline__ floatx16 load_bias(const float *b, int idx) {
 }
 
 // sin and cos of x to float rounding for |x| <= 8192 (three-constant Cody-Waite reduction by
-// pi/2, then the minimax polynomials on [-pi/4, pi/4]); callers redo larger arguments with the
+// pi/2, then polynomials on [-pi/4, pi/4]; constants and coefficients are those published with the
+// single-precision sinf / cosf of S. Moshier's Cephes library); callers redo larger arguments with the
 // library routines (kSincosMax), outside their hot loop.
 constexpr float kSincosMax = 8192.0f;
 __device__ __forceinline__ void sincos_f32(float x, float &s, float &c) {
@@ -124,13 +125,31 @@ template <int PREC> __device__ __forceinline__ bool sincos_of(float x, float &s,
     return fabsf(x) > kSincosMax;
 }
 
-// sin and cos of twice the argument.  In the fp16 modes the compiler would fold some of the conversions that follow into
-// these operations, with one rounding instead of two, here and not there: the empty asm keeps the values in fp32 first, so
-// that every kernel rounds alike.
-template <int PREC> __device__ __forceinline__ void double_angle(float s1, float c1, float &s2, float &c2) {
-    s2 = 2.0f * s1 * c1;
-    c2 = fmaf(-2.0f * s1, s1, 1.0f);
-    if (PREC == LM_MLP_F16 || PREC == LM_MLP_F16X2) asm("" : "+v"(s2), "+v"(c2));
+// sin and cos of twice the argument, for two arguments, as every kernel rounds them.  In the fp16 mode they are rounded
+// once, from the exact product straight to fp16 (the conversion that follows is exact then): left to itself the compiler does
+// so for some values in one kernel and for others in another, and rounding to fp32 first gives the wrong neighbour for one
+// value in 15 000.
+template <int PREC> __device__ __forceinline__ void double_angle(const float *s1, const float *c1, float *s2, float *c2) {
+    if constexpr (PREC == LM_MLP_F16) {
+        // In this order no instruction reads what the one before it wrote, nor a cosine that a transcendental instruction
+        // may have written right before the block (2 s1 lies between the sines and here).
+        half2v s, c;
+        asm("v_fma_mixlo_f16 %1, -%2, %3, 1.0\n\t"
+            "v_fma_mixlo_f16 %0, %2, %4, 0\n\t"
+            "v_fma_mixhi_f16 %1, -%5, %6, 1.0\n\t"
+            "v_fma_mixhi_f16 %0, %5, %7, 0"
+            : "=&v"(s), "=&v"(c)
+            : "v"(2.0f * s1[0]), "v"(s1[0]), "v"(c1[0]), "v"(2.0f * s1[1]), "v"(s1[1]), "v"(c1[1]));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { s2[i] = (float)s[i]; c2[i] = (float)c[i]; }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            s2[i] = 2.0f * s1[i] * c1[i];
+            c2[i] = fmaf(-2.0f * s1[i], s1[i], 1.0f);
+            if (PREC == LM_MLP_F16X2) asm("" : "+v"(s2[i]), "+v"(c2[i]));  // in fp32 before the split, in every kernel
+        }
+    }
 }
 
 // raw[cb][16] (the lane's 16 input rows of each of its NCB samples) -> the first layer's B fragments: per lane
@@ -145,29 +164,22 @@ __device__ __forceinline__ void encode_inputs(const float (*raw)[16],
         float slots[kSlots1];
         constexpr bool kExact = PREC == LM_MLP_F32 || PREC == LM_MLP_F16X2;
         bool big = false;
-        // row 27 / 31 (v = 15) is zero and meets zero weights
-        slots[15] = 0.0f; slots[31] = 0.0f; slots[47] = 0.0f; slots[63] = 0.0f; slots[79] = 0.0f;
 #pragma unroll
         for (int v = 0; v < 15; ++v) {
-            const float x = raw[cb][v];
-            float s1, c1;
-            big |= sincos_of<PREC>(x, s1, c1);
-            float s2, c2;
-            double_angle<PREC>(s1, c1, s2, c2);
-            slots[v] = x; slots[16 + v] = s1; slots[32 + v] = c1; slots[48 + v] = s2; slots[64 + v] = c2;
+            slots[v] = raw[cb][v];
+            big |= sincos_of<PREC>(slots[v], slots[16 + v], slots[32 + v]);
         }
+        // row 27 / 31 (v = 15) is zero and meets zero weights
+        slots[15] = 0.0f; slots[31] = 0.0f; slots[47] = 0.0f;
         if (kExact && __builtin_expect(big, 0)) {
             // arguments beyond the fast reduction's range: library routines, rarely if ever taken
 #pragma unroll
-            for (int v = 0; v < 15; ++v) {
-                const float x = raw[cb][v];
-                if (fabsf(x) > kSincosMax) {
-                    const float s1 = sinf(x), c1 = cosf(x);
-                    slots[16 + v] = s1; slots[32 + v] = c1;
-                    slots[48 + v] = 2.0f * s1 * c1; slots[64 + v] = fmaf(-2.0f * s1, s1, 1.0f);
-                }
-            }
+            for (int v = 0; v < 15; ++v)
+                if (fabsf(slots[v]) > kSincosMax) { slots[16 + v] = sinf(slots[v]); slots[32 + v] = cosf(slots[v]); }
         }
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) double_angle<PREC>(slots + 16 + v, slots + 32 + v, slots + 48 + v, slots + 64 + v);
+        slots[79] = 0.0f;
 #pragma unroll
         for (int t = 0; t < T1; ++t) M::pack(slots + t * G, bfrag[cb][t]);
     }

@@ -285,7 +285,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             }
             if (wave == 3u) s1[3] = c1[3] = 0.0f;  // row 15 of a lane is zero in every group
 #pragma unroll
-            for (int i = 0; i < 4; ++i) double_angle<PREC>(s1[i], c1[i], s2[i], c2[i]);
+            for (int i = 0; i < 4; i += 2) double_angle<PREC>(s1 + i, c1 + i, s2 + i, c2 + i);
             if (wave == 3u) c2[3] = 0.0f;
             const int v = 4 * (int)wave;
             N::write4(in1, v, lane, x);
