@@ -125,11 +125,11 @@ struct RayStats {
 // STATS: the idle lane of every quad also takes its ray's sample counts, which k_rays leaves per ray, and the workgroup
 // adds the sums to the counter block.
 template <bool STATS>
-__global__ __launch_bounds__(kBlock) void k_composite(uint64_t N, const uint32_t *__restrict__ app_first,
+__global__ __launch_bounds__(kBlock) void k_composite(uint64_t o0, uint64_t N, const uint32_t *__restrict__ app_first,
                                                            const uint32_t *__restrict__ app_cnt, const float *__restrict__ app_w,
                                                            const float *__restrict__ rgb, const float *__restrict__ acc, int white_bg,
                                                            uint32_t row, float *__restrict__ rgb_map, RayStats stats) {
-    const uint64_t o = (uint64_t)blockIdx.x * (kBlock / 4) + threadIdx.x / 4;
+    const uint64_t o = o0 + (uint64_t)blockIdx.x * (kBlock / 4) + threadIdx.x / 4;
     const unsigned ch = threadIdx.x & 3u;
     __shared__ uint32_t s_sum[2 + LM_RAY_BINS];  // samples valid and gathered, rays by their number of valid samples
     uint32_t n_valid = 0, n_marched = 0;
@@ -293,13 +293,17 @@ int lm_launch_composite(int64_t N, const uint32_t *app_first, const uint32_t *ap
                         hipStream_t stream) {
     if (N == 0) return LM_OK;
     const RayStats stats = {ray_valid, ray_marched, counters, count_valid};
-    const dim3 grid((unsigned)(((uint64_t)N + kBlock / 4 - 1) / (kBlock / 4)));
-    if (ray_valid)
-        hipLaunchKernelGGL(k_composite<true>, grid, dim3(kBlock), 0, stream, (uint64_t)N, app_first, app_cnt, app_w, rgb, acc, white_bg,
-                           row, rgb_map, stats);
-    else
-        hipLaunchKernelGGL(k_composite<false>, grid, dim3(kBlock), 0, stream, (uint64_t)N, app_first, app_cnt, app_w, rgb, acc, white_bg,
-                           row, rgb_map, stats);
+    // four threads per ray, and fewer than 2^32 threads per launch
+    constexpr uint64_t kSlice = 1ull << 29;
+    for (uint64_t o0 = 0; o0 < (uint64_t)N; o0 += kSlice) {
+        const dim3 grid((unsigned)((std::min((uint64_t)N - o0, kSlice) + kBlock / 4 - 1) / (kBlock / 4)));
+        if (ray_valid)
+            hipLaunchKernelGGL(k_composite<true>, grid, dim3(kBlock), 0, stream, o0, (uint64_t)N, app_first, app_cnt, app_w, rgb, acc,
+                               white_bg, row, rgb_map, stats);
+        else
+            hipLaunchKernelGGL(k_composite<false>, grid, dim3(kBlock), 0, stream, o0, (uint64_t)N, app_first, app_cnt, app_w, rgb, acc,
+                               white_bg, row, rgb_map, stats);
+    }
     LM_CHECK_LAUNCH("k_composite");
     return LM_OK;
 }

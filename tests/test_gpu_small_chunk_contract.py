@@ -116,3 +116,27 @@ def test_a_negative_termination_value_promises_nothing(gpu_lib, n):
         marched[term, skip] = c[L.LM_STAT_N_VALID] - c[L.LM_STAT_N_MARCHED]
     assert marched[0.0, 0] == 0 and marched[-1.0, 0] == 0
     assert marched[0.0, 1] == marched[-1.0, 1] > 0
+
+
+def test_colour_sum_of_more_rays_than_one_launch_has_threads_for(gpu_lib):
+    """lm_composite_rgb at 2^30 rays and a few: four threads per ray are more than a launch may have."""
+    n = (1 << 30) + 37
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GB of device memory")
+    cnt, first = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+    acc = torch.full((n,), 0.25, device="cuda")
+    rgb_map = torch.empty((n, 3), device="cuda")
+    w, rgb = torch.tensor([0.5, 0.25], device="cuda"), torch.tensor([[0.25, 0.5, 0.75], [0.5, 0.0, 1.0]], device="cuda")
+    at = torch.tensor([0, 1, (1 << 29) - 1, 1 << 29, (1 << 30) - 1, 1 << 30, n - 1], device="cuda")
+    cnt[at] = 2
+    L.check(gpu_lib.lm_composite_rgb(n, first.data_ptr(), cnt.data_ptr(), w.data_ptr(), rgb.data_ptr(), acc.data_ptr(), 1, rgb_map.data_ptr(),
+                                     L.current_stream()), "lm_composite_rgb")
+    torch.cuda.synchronize()
+    assert torch.equal(rgb_map[at], torch.tensor([[1.0, 1.0, 1.0]], device="cuda").expand(7, 3))
+    cnt.zero_()
+    cnt[at] = 1
+    L.check(gpu_lib.lm_composite_rgb(n, first.data_ptr(), cnt.data_ptr(), w.data_ptr(), rgb.data_ptr(), acc.data_ptr(), 0, rgb_map.data_ptr(),
+                                     L.current_stream()), "lm_composite_rgb")
+    torch.cuda.synchronize()
+    assert torch.equal(rgb_map[at], torch.tensor([[0.125, 0.25, 0.375]], device="cuda").expand(7, 3))
+    assert float(rgb_map.sum(dtype=torch.float64)) == 7 * 0.75
