@@ -42,7 +42,8 @@ def test_stopping_where_the_rest_is_lost_changes_no_bit(gpu_lib, gain, opt, S, f
     want = _render(m, rays, S, n)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and got[2:4] == want[2:4]
     assert want[4] == want[2] and got[4] <= got[2]
-    if gain >= 60.0 and thres == 1e-3 and n == 20000:  # (a small chunk's rays take 64 samples at a time)
+    # a small chunk's rays take 64 samples at a time and stop where they have more of them than that
+    if gain >= 60.0 and thres == 1e-3 and (n == 20000 or S == 300):
         assert got[4] < got[2]
 
 

@@ -701,7 +701,7 @@ def test_workspace_capacity_overflow_is_reported_and_repeatable(gpu_lib, opt, S)
 @pytest.mark.parametrize("opt,S,term,fp16,div", [(1, 128, 0.0, False, None), (1, 128, 1e-4, False, None), (0, 200, 1e-4, False, None),
                                                   (1, 64, 0.0, True, None), (0, 330, 0.0, False, None), (1, 128, 1e-4, False, (2, 3))])
 def test_both_march_kernels_give_the_same_bits(gpu_lib, opt, S, term, fp16, div):
-    """Chunks of up to 12288 rays march with a wave per ray, larger ones with a quad per ray: the same operations in
+    """Chunks of up to 12288 rays take one kernel up to the appearance list, larger ones march with a quad per ray: the same operations in
     the same order, so a ray's result does not depend on the size of the chunk it arrives in (early termination,
     word masks of long rays, fp16 tables and block-stacked tables included)."""
     from landmark_amd.render import renderer_fn
@@ -715,10 +715,10 @@ def test_both_march_kernels_give_the_same_bits(gpu_lib, opt, S, term, fp16, div)
             t.mul_(8.0)
     if fp16:
         p = O.to_fp16_features(p)
-    rays = scenes.pinhole_rays(200, 150, 170.0, scenes.sphere_pose(2.5, 9)).cuda()  # 30000 rays: one quad-march chunk
+    rays = scenes.pinhole_rays(200, 150, 170.0, scenes.sphere_pose(2.5, 9)).cuda()  # 30000 rays: one chunk of the kernels per stage
     m = _model(p, term_eps=term, mlp_precision="f16x2")
     whole, _ = renderer_fn(rays, m, chunk=1 << 20, N_samples=S, device="cuda")
-    parts, _ = renderer_fn(rays, m, chunk=7001, N_samples=S, device="cuda", exact_chunk=True)  # five wave-march chunks
+    parts, _ = renderer_fn(rays, m, chunk=7001, N_samples=S, device="cuda", exact_chunk=True)  # five small chunks
     assert float(whole["rgb_map"].min()) < 0.9
     assert torch.equal(whole["depth_map"], parts["depth_map"])
     assert torch.equal(whole["rgb_map"], parts["rgb_map"])
