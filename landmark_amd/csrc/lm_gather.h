@@ -7,7 +7,11 @@
 
 #include "lm_common.h"
 
-// chunks of up to this many rays are small: a kernel from rays to appearance entries (lm_ray.hip), or a wave per ray
+// Chunks of up to this many rays are small: a kernel from rays to appearance entries, or a wave per ray (lm_ray.hip).  The
+// line lies below where the first stops paying.  Whole calls with it / with the kernels per stage: 16384 rays of nine planes
+// 359 / 453 us, three small planes 325 / 315, 886 samples per ray 780 / 1187, 2 x 3 blocks 249 / 307, city tables 253 / 320;
+// 32768 rays 616 / 549, 509 / 427, 1469 / 1629, 430 / 396, 405 / 437; at the line itself 234 / 331, 203 / 245, 625 / 1112,
+// 148 / 227 (first four).
 #ifndef LM_RAYS_LIMIT
 #define LM_RAYS_LIMIT 12288
 #endif

@@ -139,7 +139,7 @@ __global__ __launch_bounds__(kBlock) void k_app_list(lm_geom g, PlaneSet ps, int
 // neighbouring rays are at similar depths in the same load instruction, so their corner
 // texels share cache lines; and a ray can stop once its transmittance is below term_eps,
 // before the density of the samples behind is ever fetched, or (skip_lost) once nothing behind can change its results
-// (155.8 -> 135 million samples gathered for 518400 rays of 3544 steps, 8.4 -> 6.2 million for 160000 rays of 128).  With term_eps = 0 the weights
+// (155.8 -> 129.2 million samples gathered for 518400 rays of 3544 steps, 8.4 -> 5.9 million for 160000 rays of 128).  With term_eps = 0 the weights
 // are those of the separate density + weights kernels, bit for bit (same operations, and the
 // transmittance is the same sequential product torch.cumprod forms, app/tools/utils.py:51-64).
 template <typename T, int NS>  // NS samples of a ray per round
@@ -295,8 +295,8 @@ template <int PREC> struct AppFeatBlock { static constexpr int N = 512; };
 __host__ __device__ inline size_t app_feat_tile_bytes(int C) { return (size_t)32 * (C + 4) * sizeof(float); }
 
 // XYZ: the samples are M_host points given by their normalised coordinates (`rays` = xyz[M][3]) instead of list entries.
-// Products through memory and a second kernel for basis_mat instead (k_app_xyz + k_basis) take 2.60 ms for 2^20 random
-// points of nine 48-channel planes, 1.8 GB of products written and read again; this kernel takes 1.41 ms.
+// Products through memory and a second kernel for basis_mat instead (k_app_xyz + k_basis) take 2.56 ms for 1 000 003 random
+// points of nine 48-channel planes, 1.7 GB of products written and read again; this kernel takes 1.46 ms.
 template <int PREC, typename T, int NU, bool XYZ>  // NU = groups of 16 channels per plane (C = 16 * NU)
 __global__ __launch_bounds__(AppFeatBlock<PREC>::N) void k_app_feat(lm_geom g, PlaneSet ps, int K,
                                                                    const char *__restrict__ packed, lm_mma::PackLayout L,

@@ -13,16 +13,20 @@
 //      samples that are usual at 128 samples per ray;
 //   3. the transmittance runs through a ray's samples of the round in order (the product torch.cumprod forms); the
 //      round's appearance entries are appended to the ray's list in LDS;
-//   4. one reservation per workgroup in the appearance list.  It is the only addition to the counter block: the counts per
-//      ray go to memory and the composite kernel sums them, 64 rays at a time (additions of thousands of workgroups to one
-//      line take 6.5 ns each: 12288 rays on three small planes, whole call: 232 us with
-//      valid and gathered samples added here too, 204 this way).
+//   4. one reservation per workgroup in the appearance list.  It is the only addition every workgroup makes to the counter
+//      block (dropped rays, and valid samples where they are checked against a capacity, are added too): the counts per ray
+//      go to memory and the composite kernel sums them, 64 rays at a time.  Additions of thousands of workgroups to one line
+//      take 6.5 ns each: 12288 rays on three small planes, whole call, 232 us with valid and gathered samples added here too,
+//      204 this way.
 // Four rays per workgroup: with eight the rays that see something crowd into fewer workgroups, with two or one the
 // samples of a round do not fill the waves (4096 rays of 128 samples on nine planes: 82 / 58 / 80 / 133 us with 8 / 4 / 2 /
 // 1 rays before the transmittance was spread over the lanes).
 // Measured against zeroed bitmap + cull + march with a wave per ray + list: 4096 rays as above 93 -> 45 us, 8192 rays of
 // 886 samples on three planes 393 -> 310 us, 1024 rays on three 256^2 planes 51 -> 23 us.  With skip_lost (rays
-// stop after the round behind which nothing can change their results) the second takes 229 us, the third 20.
+// stop after the round behind which nothing can change their results) the second takes 230 us, the third 18.
+// What bounds it (counters of the first / second): 3.1 / 3.8 TB/s past the L2, texture addressers 30 / 41 % busy, vector
+// ALU 28 %, 1.1 / 1.5 waves per SIMD in flight on average: latency and the longest ray of a workgroup, not bytes.
+// The fp32 instantiation holds all 256 registers and spills five (24 bytes per lane).
 // Operations and order per ray are those of the kernels for large chunks, hence the same bits.
 #include <algorithm>
 

@@ -13,8 +13,10 @@
 //      registers, requested a phase ahead; nothing is copied to LDS up front;
 //   4. one wave takes the last layer.
 // Same operations and accumulation order per sample as k_app_feat + k_mlp, hence the same bits.
-// What bounds it: with nine planes the texels (20 000 entries of 7 KB: 25 us at the rate the memory gives, 40 us taken),
-// with three small planes the chain list -> ray -> texels -> layers of one tile.  k_app_feat + k_mlp against this kernel:
+// What bounds it: with nine planes the texels (20 653 entries, 0.11 GB past the L2: 22 us at the 5.2 TB/s of a large copy, 41 us
+// taken, a third of the wave time waiting), with three small planes the chain list -> ray -> texels -> layers of one tile
+// (0.4 TB/s, addressers 15 % busy).  The split mode on 48-channel fp16 tables spills 17 registers (72 bytes per lane).
+// k_app_feat + k_mlp against this kernel:
 // 12 000 entries on three 256^2 planes, fp32 network 69 -> 25 us; 20 000 entries on nine planes, split network 74 -> 41 us;
 // 18 000 entries on three planes, a whole call 104 -> 64 us (split) and 99 -> 56 us (fp16).
 #include <algorithm>
