@@ -115,7 +115,7 @@ class GridNeRFHIP:
             if self._den_w.numel() != sum(pl.C for pl in self._density):
                 raise L.LandmarkError("basis_den width does not match the density planes")
         # rays may stop where the rest cannot change their results (lm_model.skip_lost) if the densities are finite
-        self._finite_densities = self._density_bound(torch.stack(peaks).cpu().numpy()) < 1e30 and 0.0 < float(params.distance_scale) < 1e30
+        self._finite_densities = self._density_bound(peaks) < 1e30 and 0.0 < float(params.distance_scale) < 1e30
         # --- colour network; with encode_app the 48 latent columns of the first layer fold into its bias
         self.encode_app = bool(params.encode_app)
         self._latent_dim = 0
@@ -184,7 +184,7 @@ class GridNeRFHIP:
                     self._vol_dtype, self._vol_store = L.LM_U8, as_u8.contiguous()
 
     def _relayout(self, t: torch.Tensor, peaks: Optional[list] = None) -> torch.Tensor:
-        """[1,C,H,W] -> device [H,W,C] through lm_relayout_peak; the bits of max |t| (one device word) go to `peaks`."""
+        """[1,C,H,W] -> device [H,W,C] through lm_relayout_peak; device words whose maximum holds the bits of max |t| go to `peaks`."""
         src = t.to(self.device).contiguous()
         _, Cc, H, W = src.shape
         dst = torch.empty((H, W, Cc), dtype=src.dtype, device=self.device)
@@ -194,7 +194,7 @@ class GridNeRFHIP:
             peak = torch.empty(self.lib.lm_relayout_peak_words(Cc, H, W), dtype=torch.int32, device=self.device)
         L.check(self.lib.lm_relayout_peak(src.data_ptr(), dst.data_ptr(), Cc, H, W, dt, L.ptr(peak), L.current_stream()), "relayout")
         if peaks is not None:
-            peaks.append(peak.max())
+            peaks.append(peak)
         torch.cuda.current_stream().synchronize()  # src may be a temporary
         return dst
 
@@ -230,12 +230,15 @@ class GridNeRFHIP:
         return out
 
     def _density_bound(self, peaks) -> float:
-        """Upper bound of |density feature| over all points (inf where a table holds a NaN or an infinity), from the
-        bits of the largest magnitudes, one word per table (plane, line, plane, ...)."""
+        """Upper bound of |density feature| over all points (inf where a table holds a NaN or an infinity), from the words
+        lm_relayout_peak wrote for the density tables: the largest magnitude of all of them, in one reduction."""
+        if len({pl.dtype for pl in self._density}) > 1:
+            return math.inf  # bits of different types do not compare (such planes are refused by the render)
         bound = 0.0
-        for pl, words in zip(self._density, peaks.reshape(-1, 2)):
-            top = words.view(np.float32) if pl.dtype == L.LM_F32 else words.astype(np.uint16).view(np.float16)
-            bound += pl.C * float(top[0]) * float(top[1])
+        if self._density:
+            bits = torch.cat(peaks).max().cpu().numpy()
+            top = float(bits.view(np.float32) if self._density[0].dtype == L.LM_F32 else bits.astype(np.uint16).view(np.float16))
+            bound = sum(pl.C for pl in self._density) * top * top
         if self._den_w is not None:
             bound *= float(self._den_w.abs().max())
         bound += abs(float(self.p.density_shift))

@@ -58,3 +58,32 @@ def test_tables_that_are_not_finite_keep_every_sample(gpu_lib, value):
     rays = scenes.pinhole_rays(50, 50, 45.0, scenes.sphere_pose(2.5, 9)).cuda()
     got = _render(m, rays, 128, 2500)
     assert got[4] == got[2] > 0
+
+
+def test_a_model_without_density_tables_can_still_be_asked_for_its_samples(gpu_lib):
+    """Sampling, culling, appearance lookups and the colour network need no density tables; a render without them is refused."""
+    from landmark_amd.model import GridNeRFHIP
+
+    p = _scene(60.0, 1, 128, False, 1e-3)
+    rays = scenes.pinhole_rays(20, 20, 18.0, scenes.sphere_pose(2.5, 9)).cuda()
+    want = GridNeRFHIP(p, device="cuda").sample_cull(rays)
+    p.density_plane, p.density_line = [], []
+    m = GridNeRFHIP(p, device="cuda")
+    got = m.sample_cull(rays)
+    assert torch.equal(got["ray_valid"], want["ray_valid"]) and got["n_valid"] == want["n_valid"] > 0
+    with pytest.raises(L.LandmarkError):
+        m(rays)
+    p.app_plane, p.app_line = [], []
+    with pytest.raises(L.LandmarkError):  # no colour network of width 0
+        GridNeRFHIP(p, device="cuda")
+
+
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("value,finite", [(1.0, True), (-6e4, True), (float("nan"), False), (-float("inf"), False)])
+def test_largest_magnitude_of_the_density_tables_is_found_wherever_it_lies(gpu_lib, fp16, value, finite):
+    from landmark_amd.model import GridNeRFHIP
+
+    for table, at in (("density_line", (2, (0, 15, 9, 0))), ("density_plane", (0, (0, 0, 0, 0))), ("density_plane", (2, (0, 15, 8, 6)))):
+        p = _scene(6.0, 1, 128, fp16, 1e-3)
+        getattr(p, table)[at[0]][at[1]] = value
+        assert GridNeRFHIP(p, device="cuda")._finite_densities == finite
