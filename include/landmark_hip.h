@@ -266,6 +266,12 @@ int lm_gather_density_xyz(const lm_plane *planes, int32_t n_planes, const float 
                           int64_t M, float *out, void *stream);
 int lm_gather_app_xyz(const lm_plane *planes, int32_t n_planes, const float *xyz, int64_t M, float *out,
                       void *stream);
+/* The density features of many points: with a workspace (device memory, 16-byte aligned) the points are put in the order
+ * of the planes' texels, so that every part of a table is read once.  lm_gather_density_workspace_bytes() is 0 where that
+ * does not pay or is not covered; lm_gather_density_xyz then takes the call.  The sums differ from it in rounding only. */
+size_t lm_gather_density_workspace_bytes(const lm_plane *planes, int32_t n_planes, int64_t M);
+int lm_gather_density_binned(const lm_plane *planes, int32_t n_planes, const float *density_basis, const float *xyz,
+                             int64_t M, float *out, void *workspace, size_t workspace_bytes, void *stream);
 
 /* ---- part 3: colour network ----------------------------------------------------------
  * MLPRender_Fea.forward (app/models/mlp_render_fea.py:44-68) with positional_encoding

@@ -71,6 +71,8 @@ SYMBOLS = {
     "lm_sample_cull_scratch_bytes": (_SZ, [_I64, _I32]),
     "lm_sample_cull": (C.c_int, [C.POINTER(LmGeom), _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
     "lm_gather_density_xyz": (C.c_int, [C.POINTER(LmPlane), _I32, _P, _P, _I64, _P, _P]),
+    "lm_gather_density_workspace_bytes": (_SZ, [C.POINTER(LmPlane), _I32, _I64]),
+    "lm_gather_density_binned": (C.c_int, [C.POINTER(LmPlane), _I32, _P, _P, _I64, _P, _P, _SZ, _P]),
     "lm_gather_app_xyz": (C.c_int, [C.POINTER(LmPlane), _I32, _P, _I64, _P, _P]),
     "lm_mlp_packed_bytes": (_SZ, [_I32, _I32]),
     "lm_mlp_pack": (C.c_int, [_I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P]),

@@ -750,7 +750,17 @@ class GridNeRFHIP:
         M = xyz.shape[0]
         out = torch.empty(M, dtype=torch.float32, device=self.device)
         arr = self._plane_array(self._density)
-        L.check(self.lib.lm_gather_density_xyz(arr, len(self._density), L.ptr(self._den_w), xyz.data_ptr(), M, out.data_ptr(), L.current_stream()), "lm_gather_density_xyz")
+        n, den_w, stream = len(self._density), L.ptr(self._den_w), L.current_stream()
+        need = self.lib.lm_gather_density_workspace_bytes(arr, n, M)  # many points: put in the order of the tables first
+        if need:
+            try:
+                ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+            except torch.cuda.OutOfMemoryError:
+                need = 0
+        if need:
+            L.check(self.lib.lm_gather_density_binned(arr, n, den_w, xyz.data_ptr(), M, out.data_ptr(), ws.data_ptr(), need, stream), "lm_gather_density_binned")
+        else:
+            L.check(self.lib.lm_gather_density_xyz(arr, n, den_w, xyz.data_ptr(), M, out.data_ptr(), stream), "lm_gather_density_xyz")
         return out
 
     @torch.no_grad()
