@@ -16,10 +16,6 @@
 #include "lm_gather.h"
 #include "lm_mma.h"
 
-#ifndef LM_MARCH_NS
-#define LM_MARCH_NS 4
-#endif
-
 namespace {
 
 // ---- explicit coordinates ----------------------------------------------------------------
@@ -143,7 +139,7 @@ __global__ __launch_bounds__(kBlock) void k_app_list(lm_geom g, PlaneSet ps, int
 // (155.8 -> 129.2 million samples gathered for 518400 rays of 3544 steps, 8.4 -> 5.9 million for 160000 rays of 128).  With term_eps = 0 the weights
 // are those of the separate density + weights kernels, bit for bit (same operations, and the
 // transmittance is the same sequential product torch.cumprod forms, app/tools/utils.py:51-64).
-template <typename T, int NS>  // NS samples of a ray per round
+template <typename T, int NS, bool ROLL>  // NS samples of a ray per round
 __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const float *__restrict__ den_w,
                                                   const float *__restrict__ rays, const uint64_t *__restrict__ bitmap,
                                                   const uint32_t *__restrict__ p_first,
@@ -237,7 +233,8 @@ __global__ __launch_bounds__(kBlock) void k_march(lm_geom g, PlaneSet ps, const 
                     lm_normalise(g, pt, q_m);
                     q_m[3] = __int_as_float(g.div0 > 0 ? lm_block_coords(g, q_m) : 0);
                 }
-                density_sum_n<T, NS>(ps, q_m, qlane, den_w, f);
+                if constexpr (ROLL) density_sum_rolling<T>(ps, q_m, qlane, den_w, f);
+                else density_sum_n<T, NS>(ps, q_m, qlane, den_w, f);
                 marched += (uint32_t)n_have;
                 float f_m = f[0];
 #pragma unroll
@@ -750,17 +747,17 @@ int lm_launch_march(const lm_model *m, const float *rays, const uint64_t *bitmap
     // as many workgroups as are resident at once (the kernel's register count decides), at most four per CU
     auto resident_grid = [](const void *kernel) {
         // asked once per thread and kernel: the answer depends on the kernel's registers only
-        static thread_local const void *known_on[LM_MAX_DEVICES][4] = {};
-        static thread_local unsigned grid_on[LM_MAX_DEVICES][4] = {};
+        static thread_local const void *known_on[LM_MAX_DEVICES][6] = {};
+        static thread_local unsigned grid_on[LM_MAX_DEVICES][6] = {};
         const int dev = lm_current_device();
         const void **known = known_on[dev];
         unsigned *grid = grid_on[dev];
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 6; ++i)
             if (known[i] == kernel) return grid[i];
         int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess || per_cu < 1) per_cu = 2;
         const unsigned g = (unsigned)lm_persistent_blocks(std::min(per_cu, 4));
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 6; ++i)
             if (!known[i]) { known[i] = kernel; grid[i] = g; break; }
         return g;
     };
@@ -769,22 +766,27 @@ int lm_launch_march(const lm_model *m, const float *rays, const uint64_t *bitmap
     // few rays: a wave per ray, one launch-wide round trip per 64-sample word instead of one per four samples
     if (n_rays <= LM_RAYS_LIMIT)
         return lm_launch_march_wave(m, rays, bitmap, p_first, word_mask, ray_list, bins, n_rays, w_valid, acc, depth, app_cnt, p_end, n_marched, st);
-#define LM_MARCH(T_, NS_)                                                                                              \
-    hipLaunchKernelGGL((k_march<T_, NS_>), dim3(resident_grid(reinterpret_cast<const void *>(&k_march<T_, NS_>))),         \
+#define LM_MARCH_ONE(T_, ROLL_)                                                                                            \
+    hipLaunchKernelGGL((k_march<T_, 4, ROLL_>), dim3(resident_grid(reinterpret_cast<const void *>(&k_march<T_, 4, ROLL_>))), \
                        dim3(kBlock), 0, st, m->geom, ps, m->density_basis, rays, bitmap,   \
                        p_first, word_mask, ray_list, bins, n_rays, queue, m->act, m->density_shift, m->distance_scale,            \
                        m->weight_thres, lm_stop_value(*m), w_valid, acc, depth, app_cnt, p_end, n_marched)
+#define LM_MARCH(T_)                                                                   \
+    if (density_rolls<T_>(m->density, m->n_planes, ps.nblk)) LM_MARCH_ONE(T_, true);   \
+    else LM_MARCH_ONE(T_, false)
     // Four samples per round: one per lane of the quad for the footprint arithmetic, 24 loads per lane and plane
     // in flight, half as many dependent round trips per ray as with two (1080p frame, nine fp32 planes: 2.70 ->
-    // 2.50 ms although the kernel then holds 223 registers and two waves per SIMD instead of three).
+    // 2.50 ms although the kernel then holds two waves per SIMD instead of three).  The rolling sum forced into three waves
+    // (168 registers) spills: 22.9 -> 25.6 ms on the frame of 3544 samples per ray.
     if (dtype == LM_F32) {
-        LM_MARCH(float, LM_MARCH_NS);
+        LM_MARCH(float);
     } else if (c_max <= 16) {  // 16-byte loads would leave half of every quad idle
-        LM_MARCH(Half4, 4);
+        LM_MARCH(Half4);
     } else {
-        LM_MARCH(__half, 4);
+        LM_MARCH(__half);
     }
 #undef LM_MARCH
+#undef LM_MARCH_ONE
     LM_CHECK_LAUNCH("k_march");
     return LM_OK;
 }
