@@ -351,8 +351,8 @@ __device__ __forceinline__ void density_sum_n(const PlaneSet &ps, const float *q
 // registers (all four samples' in fp32, two at a time in fp16).  Offsets are 32-bit bytes from the plane's (scalar) address:
 // a fifth of the march's vector instructions less (3.54 -> 2.83 G on the frame below) and 197 instead of 231 registers.  Same
 // operations per sample, hence the same bits.
-// 960 x 540 rays of 3544 samples, three fp32 planes with a projection: frame 26.1 -> 22.5 ms (march 13.2 -> 9.6); 8192 rays of 886
-// samples 454 -> 431 us; 4K city (fp16) 39.7 -> 39.0 ms; frames bound by bytes 1 %.  Two samples at a time in fp32 too 23.0, one
+// 960 x 540 rays of 3544 samples, three fp32 planes with a projection: frame 26.1 -> 22.5 ms (march 13.2 -> 9.6); 4K city (fp16)
+// 39.7 -> 39.0 ms; frames bound by bytes 1 %.  Two samples at a time in fp32 too 23.0, one
 // 23.5; the same without work on the next plane 24.5.  The projection's weights are loaded once per plane: once per sample is
 // what the compiler made of the plain form, and that took 30.0.
 struct RollTaps {
@@ -410,6 +410,41 @@ template <typename T> inline bool density_rolls(const lm_plane *planes, int n, i
     }
     return true;
 }
+// NS samples of a quad: lane n brings sample n's taps (NS = 1: every lane its own sample's).  A lane beyond a narrow plane's
+// channels reads its last ones and adds nothing.
+template <typename T> __device__ __forceinline__ int roll_channel(const lm_plane &pl, unsigned qlane) { return min(Vec<T>::V * (int)qlane, pl.C - Vec<T>::V); }
+template <typename T, int NS>
+__device__ __forceinline__ void roll_load(const lm_plane &pl, const RollTaps &m, int n, unsigned qlane, Footprint<T> &f) {
+    auto of = [&](uint32_t v) { return NS == 1 ? v : (uint32_t)quad_lane((int)v, n); };
+    const uint32_t c = (uint32_t)(roll_channel<T>(pl, qlane) * (int)sizeof(typename Vec<T>::elem));
+    const uint32_t o00 = of(m.o00) + c, dx = of(m.dx), dy = of(m.dy), l0 = of(m.l0) + c, dl = of(m.dl), o10 = o00 + dy;
+    f.a = fetch_at<T>(pl.plane, o00);
+    f.b = fetch_at<T>(pl.plane, o00 + dx);
+    f.c = fetch_at<T>(pl.plane, o10);
+    f.d = fetch_at<T>(pl.plane, o10 + dx);
+    f.l0 = fetch_at<T>(pl.line, l0);
+    f.l1 = fetch_at<T>(pl.line, l0 + dl);
+}
+template <typename T> __device__ __forceinline__ void roll_weights(const lm_plane &pl, const float *__restrict__ den_w, int col, unsigned qlane, float *w) {
+    if (!den_w) return;
+#pragma unroll
+    for (int i = 0; i < Vec<T>::V; ++i) w[i] = den_w[col + roll_channel<T>(pl, qlane) + i];
+}
+template <typename T, int NS>
+__device__ __forceinline__ void roll_use(const lm_plane &pl, const RollTaps &m, int n, unsigned qlane, const Footprint<T> &f, bool weighted, const float *w,
+                                         float &sum) {
+    constexpr int V = Vec<T>::V;
+    auto of = [&](float v) { return NS == 1 ? v : quad_lane(v, n); };
+    Taps2 t2;
+    Taps1 t1;
+    t2.w00 = of(m.w00); t2.w01 = of(m.w01); t2.w10 = of(m.w10); t2.w11 = of(m.w11);
+    t1.w0 = of(m.lw0); t1.w1 = of(m.lw1);
+    float prod[V];
+    footprint_products<T>(f, t2, t1, prod);
+    if (V * (int)qlane >= pl.C) return;
+#pragma unroll
+    for (int i = 0; i < V; ++i) sum = weighted ? fmaf(w[i], prod[i], sum) : sum + prod[i];
+}
 template <typename T>
 __device__ __forceinline__ void density_sum_rolling(const PlaneSet &ps, const float *q_mine, unsigned qlane, const float *__restrict__ den_w,
                                                     float *out) {
@@ -419,41 +454,12 @@ __device__ __forceinline__ void density_sum_rolling(const PlaneSet &ps, const fl
 #pragma unroll
     for (int n = 0; n < NS; ++n) sum[n] = 0.0f;
     Footprint<T> f[NS];
-    // a lane beyond a narrow plane's channels reads its last ones and adds nothing
-    auto channel = [&](const lm_plane &pl) { return min(V * (int)qlane, pl.C - V); };
-    auto load = [&](const lm_plane &pl, const RollTaps &m, int n) {
-        const uint32_t c = (uint32_t)(channel(pl) * (int)sizeof(E));
-        const uint32_t o00 = (uint32_t)quad_lane((int)m.o00, n) + c, dx = (uint32_t)quad_lane((int)m.dx, n), dy = (uint32_t)quad_lane((int)m.dy, n);
-        const uint32_t l0 = (uint32_t)quad_lane((int)m.l0, n) + c, dl = (uint32_t)quad_lane((int)m.dl, n), o10 = o00 + dy;
-        f[n].a = fetch_at<T>(pl.plane, o00);
-        f[n].b = fetch_at<T>(pl.plane, o00 + dx);
-        f[n].c = fetch_at<T>(pl.plane, o10);
-        f[n].d = fetch_at<T>(pl.plane, o10 + dx);
-        f[n].l0 = fetch_at<T>(pl.line, l0);
-        f[n].l1 = fetch_at<T>(pl.line, l0 + dl);
-    };
-    auto weights = [&](const lm_plane &pl, int col, float *w) {
-        if (!den_w) return;
-#pragma unroll
-        for (int i = 0; i < V; ++i) w[i] = den_w[col + channel(pl) + i];
-    };
-    auto use = [&](const lm_plane &pl, const RollTaps &m, int n, const float *w) {
-        Taps2 t2;
-        Taps1 t1;
-        t2.w00 = quad_lane(m.w00, n); t2.w01 = quad_lane(m.w01, n); t2.w10 = quad_lane(m.w10, n); t2.w11 = quad_lane(m.w11, n);
-        t1.w0 = quad_lane(m.lw0, n); t1.w1 = quad_lane(m.lw1, n);
-        float prod[V];
-        footprint_products<T>(f[n], t2, t1, prod);
-        if (V * (int)qlane >= pl.C) return;
-#pragma unroll
-        for (int i = 0; i < V; ++i) sum[n] = den_w ? fmaf(w[i], prod[i], sum[n]) : sum[n] + prod[i];
-    };
     lm_plane pl = ps.p[0];
     RollTaps now = roll_taps<E>(pl, ps.nblk, q_mine);
     float w[V] = {}, w_next[V] = {};
-    weights(pl, 0, w);
+    roll_weights<T>(pl, den_w, 0, qlane, w);
 #pragma unroll
-    for (int n = 0; n < NS; ++n) load(pl, now, n);
+    for (int n = 0; n < NS; ++n) roll_load<T, NS>(pl, now, n, qlane, f[n]);
     int col = 0;
     for (int k = 0;;) {
         const bool last = k + 1 == ps.n;
@@ -465,12 +471,12 @@ __device__ __forceinline__ void density_sum_rolling(const PlaneSet &ps, const fl
         for (int h = 0; h < NS; h += HALF) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int n = h; n < h + HALF; ++n) use(pl, now, n, w);
+            for (int n = h; n < h + HALF; ++n) roll_use<T, NS>(pl, now, n, qlane, f[n], den_w != nullptr, w, sum[n]);
             __builtin_amdgcn_sched_barrier(0);
             if (!last) {
-                if (h == 0) weights(pn, col + pl.C, w_next);
+                if (h == 0) roll_weights<T>(pn, den_w, col + pl.C, qlane, w_next);
 #pragma unroll
-                for (int n = h; n < h + HALF; ++n) load(pn, next, n);
+                for (int n = h; n < h + HALF; ++n) roll_load<T, NS>(pn, next, n, qlane, f[n]);
             }
         }
         if (last) break;

@@ -8,8 +8,7 @@
 //      level).  Lane = sample: the decisions of those words, four words' lookups in flight, kept in LDS;
 //   2. rounds: every ray contributes its next (up to) 64 valid samples, ascending.  The round's samples are dealt evenly
 //      to the four waves and gathered four lanes to a sample.  Up to 16 samples per wave give every quad one sample and
-//      three planes at a time, up to 32 two samples and two planes, more four samples and one plane at a time,
-//      with the next one's loads issued ahead: about 24 loads per
+//      three planes at a time, up to 32 two samples and two planes, more four samples and one plane: about 24 loads per
 //      lane in flight either way, and nine planes are three round trips instead of nine for the rays with a dozen valid
 //      samples that are usual at 128 samples per ray;
 //   3. the transmittance runs through a ray's samples of the round in order (the product torch.cumprod forms); the
@@ -27,7 +26,9 @@
 // stop after the round behind which nothing can change their results) the second takes 230 us, the third 18.
 // What bounds it (counters of the first / second): 3.1 / 3.8 TB/s past the L2, texture addressers 30 / 41 % busy, vector
 // ALU 28 %, 1.1 / 1.5 waves per SIMD in flight on average: latency and the longest ray of a workgroup, not bytes.
-// The fp32 instantiation holds all 256 registers and spills nine (40 bytes per lane).
+// With 32-bit offsets and only the weights of the taps kept (density_sum_lean, tables below 4 GB) the fp32 kernel holds 210 registers
+// instead of 256 and five spilled: 1024 rays 51.0 -> 48.4 us, 4096 rays 108.4 -> 104.2, 8192 rays of 886 samples 454 -> 419 (whole
+// calls).  Forced into three waves per SIMD (168 registers, 30 spilled) 4096 rays take 126.
 // Operations and order per ray are those of the kernels for large chunks, hence the same bits.
 #include <algorithm>
 
@@ -94,9 +95,49 @@ __device__ __forceinline__ void density_sum_planes(const PlaneSet &ps, const flo
     }
 }
 
-template <typename T>
+// The same for tables density_sum_rolling takes: 32-bit offsets that are used up by the loads, and of the taps only the weights
+// kept (on the lane that worked them out).  Same operations per sample, hence the same bits.
+template <typename T, int NS, int G>
+__device__ __forceinline__ void density_sum_lean(const PlaneSet &ps, const float *q_mine, unsigned qlane, const float *__restrict__ den_w, float *out) {
+    float sum[NS];
+#pragma unroll
+    for (int n = 0; n < NS; ++n) sum[n] = 0.0f;
+    int col = 0;
+    for (int k0 = 0; k0 < ps.n; k0 += G) {
+        RollTaps m[G];
+        Footprint<T> f[G][NS];
+        float w[G][Vec<T>::V] = {};
+        int at = col;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            if (k0 + i >= ps.n) break;
+            const lm_plane pl = ps.p[k0 + i];
+            m[i] = roll_taps<typename Vec<T>::elem>(pl, ps.nblk, q_mine);
+            roll_weights<T>(pl, den_w, at, qlane, w[i]);
+            at += pl.C;
+#pragma unroll
+            for (int n = 0; n < NS; ++n) roll_load<T, NS>(pl, m[i], n, qlane, f[i][n]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            if (k0 + i >= ps.n) break;
+            const lm_plane pl = ps.p[k0 + i];
+#pragma unroll
+            for (int n = 0; n < NS; ++n) roll_use<T, NS>(pl, m[i], n, qlane, f[i][n], den_w != nullptr, w[i], sum[n]);
+        }
+        col = at;
+    }
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+        const float v = quad_sum(sum[n]);
+        out[n] = den_w ? fmaxf(v, 0.0f) : v;
+    }
+}
+
+template <typename T, bool ROLL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_rays(
-    lm_geom g, PlaneSet ps, int narrow, int rolls, const float *__restrict__ den_w, const float *__restrict__ rays, uint32_t N, uint32_t row,
+    lm_geom g, PlaneSet ps, int narrow, const float *__restrict__ den_w, const float *__restrict__ rays, uint32_t N, uint32_t row,
     int ent, int act, float shift, float distance_scale, float weight_thres, float stop, uint32_t cap_valid,
     uint32_t *__restrict__ app_first, uint32_t *__restrict__ app_cnt, uint32_t *__restrict__ app_idx, float *__restrict__ app_w,
     uint32_t cap_app, float *__restrict__ acc_out, float *__restrict__ depth_out, uint32_t *__restrict__ ray_valid,
@@ -238,8 +279,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             lm_point(ray, z_m, pt);
             lm_normalise(g, pt, q_m);
             q_m[3] = __int_as_float(g.div0 > 0 ? lm_block_coords(g, q_m) : 0);
-            if constexpr (G > 1) density_sum_planes<T, NS, G>(ps, q_m, qlane, den_w, d);
-            else if constexpr (G == 0) density_sum_rolling<T>(ps, q_m, qlane, den_w, d);
+            if constexpr (ROLL) density_sum_lean<T, NS, G>(ps, q_m, qlane, den_w, d);
+            else if constexpr (G > 1) density_sum_planes<T, NS, G>(ps, q_m, qlane, den_w, d);
             else density_sum_n<T, NS>(ps, q_m, qlane, den_w, d);
             float d_m = d[0];
 #pragma unroll
@@ -255,9 +296,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             }
         };
         using std::integral_constant;
-        if (narrow && share <= 16u) batch(integral_constant<int, 1>{}, integral_constant<int, 3>{});
-        else if (narrow && share <= 32u) batch(integral_constant<int, 2>{}, integral_constant<int, 2>{});
-        else if (rolls) batch(integral_constant<int, 4>{}, integral_constant<int, 0>{});
+        if ((ROLL || narrow) && share <= 16u) batch(integral_constant<int, 1>{}, integral_constant<int, 3>{});
+        else if ((ROLL || narrow) && share <= 32u) batch(integral_constant<int, 2>{}, integral_constant<int, 2>{});
         else batch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
         __syncthreads();
         // Transmittance of the wave's own ray.  Only the three running values are a chain: lane 0 multiplies its way
@@ -489,16 +529,23 @@ int lm_launch_rays(const lm_model *m, const float *rays, uint32_t N, uint32_t ro
     for (int k = 0; k < m->n_planes; ++k) c_max = std::max(c_max, (int)m->density[k].C);
     const int ent = std::min(m->geom.S, kEntriesMax);
     const size_t lds = (size_t)kRays * ent * (sizeof(float) + sizeof(uint16_t));
-#define LM_RAYS(T_)                                                                                                           \
-    hipLaunchKernelGGL((k_rays<T_>), dim3((N + kRays - 1) / kRays), dim3(kBlock), lds, st, m->geom, ps, c_max <= Vec<T_>::V * kQuad ? 1 : 0, \
-                       density_rolls<T_>(m->density, m->n_planes, ps.nblk) ? 1 : 0,                                            \
+#define LM_RAYS_ONE(T_, ROLL_)                                                                                                \
+    hipLaunchKernelGGL((k_rays<T_, ROLL_>), dim3((N + kRays - 1) / kRays), dim3(kBlock), lds, st, m->geom, ps, c_max <= Vec<T_>::V * kQuad ? 1 : 0, \
                        m->density_basis, rays, N, row, ent, m->act, m->density_shift, m->distance_scale, m->weight_thres,    \
                        lm_stop_value(*m), cap_valid, app_first, app_cnt, app_idx, app_w, cap_app, acc, depth, ray_valid,       \
                        ray_marched, counters)
-    if (dtype == LM_F32) LM_RAYS(float);
-    else if (c_max <= 16) LM_RAYS(Half4);
-    else LM_RAYS(__half);
+#define LM_RAYS(T_)                                                                  \
+    if (density_rolls<T_>(m->density, m->n_planes, ps.nblk)) LM_RAYS_ONE(T_, true);  \
+    else LM_RAYS_ONE(T_, false)
+    if (dtype == LM_F32) {
+        LM_RAYS(float);
+    } else if (c_max <= 16) {
+        LM_RAYS(Half4);
+    } else {
+        LM_RAYS(__half);
+    }
 #undef LM_RAYS
+#undef LM_RAYS_ONE
     LM_CHECK_LAUNCH("k_rays");
     return LM_OK;
 }
