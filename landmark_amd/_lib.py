@@ -88,6 +88,7 @@ SYMBOLS = {
     "lm_app_features": (C.c_int, [C.POINTER(LmModel), _P, _P, _P, _P, _P]),
     "lm_render_route": (C.c_int, [C.POINTER(LmModel), _I64]),
     "lm_render": (C.c_int, [C.POINTER(LmModel), _P, _I64, _P, _SZ, _P, _P, _P, _P]),
+    "lm_render_chunks": (C.c_int, [C.POINTER(LmModel), _P, _I64, _I64, _I32, C.POINTER(_P), C.POINTER(_P), C.POINTER(_SZ), _P, _P, _P]),
     "lm_render_static": (C.c_int, [C.POINTER(LmModel), _P, _I64, _P, _P, _P, _P]),
     "lm_generate_rays": (C.c_int, [_P, _P, _P, _I32, _I32, _P, _P]),
     "lm_rgba8": (C.c_int, [_P, _I64, _P, _P]),

@@ -213,7 +213,7 @@ int check_model(const lm_model *m, int *K) {
 }
 
 int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *workspace, size_t workspace_bytes,
-                 float *rgb_map, float *depth_map, uint32_t *counters, void *stream);
+                 float *rgb_map, float *depth_map, uint32_t *counters, bool clear, void *stream);
 }  // namespace
 
 extern "C" size_t lm_render_workspace_bytes(const lm_model *m, int64_t N) {
@@ -235,7 +235,25 @@ extern "C" int lm_render(const lm_model *m, const float *rays, int64_t N, void *
                          float *rgb_map, float *depth_map, uint32_t *counters, void *stream) {
     int K;
     if (int rc = check_model(m, &K)) return rc;
-    return render_chunk(m, K, rays, N, workspace, workspace_bytes, rgb_map, depth_map, counters, stream);
+    return render_chunk(m, K, rays, N, workspace, workspace_bytes, rgb_map, depth_map, counters, true, stream);
+}
+
+extern "C" int lm_render_chunks(const lm_model *m, const float *rays, int64_t N, int64_t step, int32_t n_streams, void *const *streams,
+                                void *const *workspaces, const size_t *workspace_bytes, float *rgb_map, float *depth_map,
+                                uint32_t *counters) {
+    int K;
+    if (int rc = check_model(m, &K)) return rc;
+    LM_REQUIRE(N >= 0 && step > 0, "negative ray count or no rays per chunk");
+    if (N == 0) return LM_OK;
+    LM_REQUIRE(n_streams > 0 && streams && workspaces && workspace_bytes && rays && rgb_map && depth_map && counters, "null buffer or no stream");
+    int64_t i = 0;
+    for (int64_t at = 0; at < N; at += step, ++i) {
+        const int32_t s = (int32_t)(i % n_streams);
+        if (int rc = render_chunk(m, K, rays + 6 * at, std::min(step, N - at), workspaces[s], workspace_bytes[s], rgb_map + 3 * at, depth_map + at,
+                                  counters + i * LM_STAT_WORDS, false, streams[s]))
+            return rc;
+    }
+    return LM_OK;
 }
 
 // ---- the same render out of a workspace that lives in the library's own image ------------------
@@ -282,12 +300,13 @@ extern "C" int lm_render_static(const lm_model *m, const float *rays, int64_t N,
                 (long long)N, m->geom.S, need, (size_t)LM_STATIC_WORKSPACE_BYTES);
     void *ws = nullptr;
     if (int rc = static_workspace(&ws)) return rc;
-    return render_chunk(m, K, rays, N, ws, (size_t)LM_STATIC_WORKSPACE_BYTES, rgb_map, depth_map, counters, stream);
+    return render_chunk(m, K, rays, N, ws, (size_t)LM_STATIC_WORKSPACE_BYTES, rgb_map, depth_map, counters, true, stream);
 }
 
 namespace {
+// clear: the counter block is cleared here (else the caller has done so)
 int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *workspace, size_t workspace_bytes,
-                 float *rgb_map, float *depth_map, uint32_t *counters, void *stream) {
+                 float *rgb_map, float *depth_map, uint32_t *counters, bool clear, void *stream) {
     LM_REQUIRE(N >= 0, "negative ray count");
     if (N == 0) return LM_OK;
     LM_REQUIRE(rays && rgb_map && depth_map, "null buffer");
@@ -308,7 +327,8 @@ int render_chunk(const lm_model *m, int K, const float *rays, int64_t N, void *w
     LM_REQUIRE(m->ray_row >= 0, "negative ray_row");
     const uint32_t row = m->ray_row % 8 == 0 ? (uint32_t)m->ray_row : 0u;  // tiles of 8 x 8 pixels need whole tiles per row
     mark(0);
-    if (int rc = lm_launch_zero_counters(cnt, st)) return rc;
+    if (clear)
+        if (int rc = lm_launch_zero_counters(cnt, st)) return rc;
     const bool few = lm_rays_kernel_takes(m, N);
     if (few) {
         // few rays: one kernel up to the appearance list (p_first, p_end: samples valid and gathered per ray)
