@@ -196,6 +196,7 @@ __device__ __forceinline__ void dense_layer(const typename Mma<PREC>::frag *W0, 
                 for (int pt = 0; pt < NP; ++pt) a[t + PF][fb][pt] = W[((fb * T + t + PF) * NP + pt) * 64];
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (M::G == 1 && T == kSlots1 && t % 16 == 15) continue;  // rows 27 and 31 of a group: zero inputs, zero weights
 #pragma unroll
         for (int fb = 0; fb < NB; ++fb)
 #pragma unroll
@@ -253,10 +254,23 @@ __device__ __forceinline__ void colour_layers(const typename Mma<PREC>::frag *w1
 #pragma unroll
             for (int cb = 0; cb < NCB; ++cb) relu_to_frags<PREC>(acc[fb][cb], &b3frag[cb][(pass * NB + fb) * (16 / G)]);
     }
+    if constexpr (PREC == LM_MLP_F32) {
+        // w3: {row 0, row 1, row 2, 0} of every slot, both halves (stage_weights)
+        const float4 *w = reinterpret_cast<const float4 *>(w3) + h;
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            float part[4][3];
+#pragma unroll
+            for (int fb = 0; fb < 4; ++fb) last_layer_block(&b3frag[cb][fb * 16][0], [&](int v) { return w[2 * (fb * 16 + v)]; }, part[fb]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) out[cb][k] = colour_of<PREC>(last_layer_sum(part[0][k], part[1][k], part[2][k], part[3][k], b3[k]));
+        }
+        return;
+    }
     floatx16 acc3[1][NCB];
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) acc3[0][cb] = load_bias(b3, h);
-    dense_layer<PREC, 1, NCB, T2, (G == 1 ? 8 : 4)>(w3, 0, lane, b3frag, acc3);
+    dense_layer<PREC, 1, NCB, T2, 4>(w3, 0, lane, b3frag, acc3);
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
@@ -373,8 +387,9 @@ template <int PREC> struct LdsPlan {
     using M = Mma<PREC>;
     static constexpr size_t kW1 = (size_t)4 * kSlots1 * 64 * sizeof(typename M::elem) * M::NP;
     static constexpr size_t kW2 = (size_t)4 * 64 * 64 * sizeof(typename M::elem) * M::NP;
-    static constexpr size_t kW3 = (size_t)64 * 64 * sizeof(typename M::elem) * M::NP;
-    static constexpr bool kW3InLds = (kW1 + kW2 + kW3) <= 96 * 1024;
+    // fp32: the three rows in use only, as four floats per slot and half (last_layer_block)
+    static constexpr size_t kW3 = PREC == LM_MLP_F32 ? (size_t)64 * 2 * 16 : (size_t)64 * 64 * sizeof(typename M::elem) * M::NP;
+    static constexpr bool kW3InLds = PREC == LM_MLP_F32 || (kW1 + kW2 + kW3) <= 96 * 1024;
     static constexpr size_t kBias = (4 * 2 * 16 + 4 * 2 * 16 + 2 * 16) * sizeof(float);  // b1 | b2 | b3, register order
     static constexpr size_t kWeights = kW1 + kW2 + (kW3InLds ? kW3 : 0);
     static constexpr size_t kQueue = kWeights + kBias;  // the workgroup's tile counter
@@ -399,8 +414,11 @@ __device__ __forceinline__ void stage_weights(char *lds, const char *packed, con
     d += P::kW1 / 16;
     for (size_t i = threadIdx.x; i < P::kW2 / 16; i += blockDim.x) d[i] = s2[i];
     d += P::kW2 / 16;
-    if (P::kW3InLds)
+    if constexpr (PREC == LM_MLP_F32) {
+        for (size_t i = threadIdx.x; i < P::kW3 / 16; i += blockDim.x) d[i] = s3[i * 8];  // slot i / 2, half i % 2: 32 rows each
+    } else if (P::kW3InLds) {
         for (size_t i = threadIdx.x; i < P::kW3 / 16; i += blockDim.x) d[i] = s3[i];
+    }
     // biases: read once per layer and row block by every wave, so they live next to the weights
     float *bl = reinterpret_cast<float *>(lds + P::kWeights);
     const float *b1 = (const float *)(packed + L.b1), *b2 = (const float *)(packed + L.b2), *b3 = (const float *)(packed + L.b3);

@@ -11,14 +11,15 @@
 //   3. every wave encodes the 32 inputs and takes one of the four row blocks of layers 1 and 2; activations go through
 //      LDS once per layer.  Each wave needs a weight fragment once per tile, so fragments come straight from the L2 into
 //      registers, requested a phase ahead; nothing is copied to LDS up front;
-//   4. one wave takes the last layer.
+//   4. one wave takes the last layer; in fp32 every wave its row block's share on the vector unit, and one adds them up.
 // Same operations and accumulation order per sample as k_app_feat + k_mlp, hence the same bits.
 // What bounds it: with nine planes the texels (20 653 entries, 0.11 GB past the L2: 22 us at the 5.2 TB/s of a large copy, 41 us
 // taken, a third of the wave time waiting), with three small planes the chain list -> ray -> texels -> layers of one tile
 // (0.4 TB/s, addressers 15 % busy).  The split mode on 48-channel fp16 tables spills 17 registers (72 bytes per lane).
 // k_app_feat + k_mlp against this kernel:
-// 12 000 entries on three 256^2 planes, fp32 network 69 -> 25 us; 20 000 entries on nine planes, split network 74 -> 41 us;
-// 18 000 entries on three planes, a whole call 104 -> 64 us (split) and 99 -> 56 us (fp16).
+// 12 000 entries on three 256^2 planes, fp32 network 69 -> 25 us (22 with the last layer's three rows on the vector unit);
+// 20 000 entries on nine planes, split network 74 -> 41 us; 18 000 entries on three planes, a whole call 104 -> 64 us (split)
+// and 99 -> 56 us (fp16).
 #include <algorithm>
 
 #include "lm_colour.h"
@@ -306,7 +307,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
             for (int i = 0; i < N::S; ++i) {
                 const int t = u * N::S + i;
-                acc = step(wa[t], x[i], acc);
+                if (!(G == 1 && t % 16 == 15)) acc = step(wa[t], x[i], acc);  // (rows 27 and 31: zero inputs, zero weights)
                 if (t >= T1 - T2) {
 #pragma unroll
                     for (int pt = 0; pt < NP; ++pt) wb[t - (T1 - T2)][pt] = weight(w2, (t - (T1 - T2)) * NP + pt, here);
@@ -320,6 +321,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         publish(in2);
         acc = bias_of(L.b2 + wave * 128u, bias);
         __syncthreads();
+        // (fp32: the wave's rows of layer 3 travel meanwhile)
+        float4 w3[G == 1 ? 16 : 1];
+        if constexpr (G == 1) {
+            const uint32_t half = (here / (uint32_t)sizeof(frag) / 32u) * 128u;
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                w3[v] = *reinterpret_cast<const float4 *>(packed + L.w3 + (size_t)(wave * 16 + v) * (LM_WAVE * sizeof(float)) + half);
+        }
         // ---- layer 2
 #pragma unroll
         for (int u = 0; u < N::U2; ++u) {
@@ -328,30 +337,56 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
             for (int i = 0; i < N::S; ++i) acc = step(wb[u * N::S + i], x[i], acc);
         }
-        frag wc[T2][NP];
-        if (wave == kLead) {
+        if constexpr (G == 1) {
+            // ---- layer 3 in fp32: every wave its own row block's share of the three outputs, one wave adds them up
+            float x[16], part[3];
 #pragma unroll
-            for (int t = 0; t < T2; ++t)
+            for (int v = 0; v < 16; ++v) x[v] = relu_f32(acc[v]);
+            last_layer_block(x, [&](int v) { return w3[v]; }, part);
+            float *sums = reinterpret_cast<float *>(in3);  // (layer 1's inputs are done with: every wave is past layer 1)
 #pragma unroll
-                for (int pt = 0; pt < NP; ++pt) wc[t][pt] = weight(L.w3, t * NP + pt, here);
-        }
-        publish(in3);
-        position(gn, vn);
-        __syncthreads();
-        // ---- layer 3
-        if (wave == kLead) {
-            acc = bias_of(L.b3, bias);
+            for (int k = 0; k < 3; ++k) sums[(wave * 3 + k) * LM_WAVE + lane] = part[k];
+            position(gn, vn);
+            __syncthreads();
+            if (wave == kLead) {
+                const float *b3 = reinterpret_cast<const float *>(packed + L.b3);
+                const uint32_t p = tile * kTileRays + j;
+                float out[3];
 #pragma unroll
-            for (int u = 0; u < N::U2; ++u) {
-                frag x[N::S][NP];
-                N::read(in3 + u * N::kBytes, lane, x);
+                for (int k = 0; k < 3; ++k)
+                    out[k] = last_layer_sum(sums[k * LM_WAVE + lane], sums[(3 + k) * LM_WAVE + lane], sums[(6 + k) * LM_WAVE + lane],
+                                            sums[(9 + k) * LM_WAVE + lane], b3[k]);
+                if (p < M && h == 0) {
 #pragma unroll
-                for (int i = 0; i < N::S; ++i) acc = step(wc[u * N::S + i], x[i], acc);
+                    for (int i = 0; i < 3; ++i) rgb[(size_t)p * 3 + i] = colour_of<PREC>(out[i]);
+                }
             }
-            const uint32_t p = tile * kTileRays + j;
-            if (p < M && h == 0) {
+        } else {
+            frag wc[T2][NP];
+            if (wave == kLead) {
 #pragma unroll
-                for (int i = 0; i < 3; ++i) rgb[(size_t)p * 3 + i] = colour_of<PREC>(acc[i]);
+                for (int t = 0; t < T2; ++t)
+#pragma unroll
+                    for (int pt = 0; pt < NP; ++pt) wc[t][pt] = weight(L.w3, t * NP + pt, here);
+            }
+            publish(in3);
+            position(gn, vn);
+            __syncthreads();
+            // ---- layer 3
+            if (wave == kLead) {
+                acc = bias_of(L.b3, bias);
+#pragma unroll
+                for (int u = 0; u < N::U2; ++u) {
+                    frag x[N::S][NP];
+                    N::read(in3 + u * N::kBytes, lane, x);
+#pragma unroll
+                    for (int i = 0; i < N::S; ++i) acc = step(wc[u * N::S + i], x[i], acc);
+                }
+                const uint32_t p = tile * kTileRays + j;
+                if (p < M && h == 0) {
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) rgb[(size_t)p * 3 + i] = colour_of<PREC>(acc[i]);
+                }
             }
         }
         __syncthreads();  // the next tile's products overwrite layer 3's inputs
