@@ -547,48 +547,50 @@ class GridNeRFHIP:
         starts = list(range(0, N, step))
         if not starts:
             return 0
-        current = torch.cuda.current_stream(self.device)
-        side = self.side_streams(min(int(streams), len(starts)) - 1) if streams > 1 and len(starts) > 1 else []
-        counters = torch.zeros((len(starts), L.LM_STAT_WORDS), dtype=torch.int32, device=self.device)  # a block per chunk
-        if side:
-            ready = torch.cuda.Event()
-            ready.record(current)
+        # the library launches on the current device (and asks it for its size): that has to be the model's, whatever the caller's is
+        with torch.cuda.device(self.device):
+            current = torch.cuda.current_stream()
+            side = self.side_streams(min(int(streams), len(starts)) - 1) if streams > 1 and len(starts) > 1 else []
+            counters = torch.zeros((len(starts), L.LM_STAT_WORDS), dtype=torch.int32, device=self.device)  # a block per chunk
+            if side:
+                ready = torch.cuda.Event()
+                ready.record(current)
+                for s in side:
+                    s.wait_event(ready)
+            lanes = [current] + side
+            # the chunks of full size in one call of the library: launching them one by one from here takes 30 us each, longer
+            # than a chunk of a few thousand rays takes the GPU (960 x 540 rays in chunks of 1024: 15.6 -> 5.1
+            # ms; of 4096: 3.99 -> 3.77, the GPU is then the limit)
+            full = N // step
+            done = []
+            if full:
+                caps = self.capacities(step, S)
+                ws = []
+                for i, lane in enumerate(lanes[:full]):
+                    with torch.cuda.stream(lane):
+                        ws.append(self.workspace(step, S, i, caps))
+                n = len(ws)
+                L.check(
+                    self.lib.lm_render_chunks(
+                        C.byref(self._model_struct(S, white_bg, caps)), rays.data_ptr(), full * step, step, n,
+                        (C.c_void_p * n)(*[lane.cuda_stream for lane in lanes[:n]]), (C.c_void_p * n)(*[w.data_ptr() for w in ws]),
+                        (C.c_size_t * n)(*[w.numel() for w in ws]), rgb.data_ptr(), depth.data_ptr(), counters.data_ptr(),
+                    ),
+                    "lm_render_chunks",
+                )
+                if caps != (0, 0):
+                    done = [(slice(i * step, (i + 1) * step), counters[i], caps) for i in range(full)]
+            if full < len(starts):
+                sl = slice(full * step, N)
+                with torch.cuda.stream(lanes[full % len(lanes)]):
+                    caps = self.render_into(rays[sl], rgb[sl], depth[sl], white_bg=white_bg, N_samples=N_samples, slot=full % len(lanes),
+                                            counters=counters[full])
+                done.append((sl, counters[full], caps))
             for s in side:
-                s.wait_event(ready)
-        lanes = [current] + side
-        # the chunks of full size in one call of the library: launching them one by one from here takes 30 us each, longer
-        # than a chunk of a few thousand rays takes the GPU (960 x 540 rays in chunks of 1024: 15.6 -> 5.1
-        # ms; of 4096: 3.99 -> 3.77, the GPU is then the limit)
-        full = N // step
-        done = []
-        if full:
-            caps = self.capacities(step, S)
-            ws = []
-            for i, lane in enumerate(lanes[:full]):
-                with torch.cuda.stream(lane):
-                    ws.append(self.workspace(step, S, i, caps))
-            n = len(ws)
-            L.check(
-                self.lib.lm_render_chunks(
-                    C.byref(self._model_struct(S, white_bg, caps)), rays.data_ptr(), full * step, step, n,
-                    (C.c_void_p * n)(*[lane.cuda_stream for lane in lanes[:n]]), (C.c_void_p * n)(*[w.data_ptr() for w in ws]),
-                    (C.c_size_t * n)(*[w.numel() for w in ws]), rgb.data_ptr(), depth.data_ptr(), counters.data_ptr(),
-                ),
-                "lm_render_chunks",
-            )
-            if caps != (0, 0):
-                done = [(slice(i * step, (i + 1) * step), counters[i], caps) for i in range(full)]
-        if full < len(starts):
-            sl = slice(full * step, N)
-            with torch.cuda.stream(lanes[full % len(lanes)]):
-                caps = self.render_into(rays[sl], rgb[sl], depth[sl], white_bg=white_bg, N_samples=N_samples, slot=full % len(lanes),
-                                        counters=counters[full])
-            done.append((sl, counters[full], caps))
-        for s in side:
-            current.wait_stream(s)
-        self.finish_chunks(done, rays, rgb, depth, white_bg=white_bg, N_samples=N_samples)
-        self.counters.copy_(counters[len(starts) - 1])
-        return len(starts)
+                current.wait_stream(s)
+            self.finish_chunks(done, rays, rgb, depth, white_bg=white_bg, N_samples=N_samples)
+            self.counters.copy_(counters[len(starts) - 1])
+            return len(starts)
 
     __call__ = forward
 
