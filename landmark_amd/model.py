@@ -563,31 +563,33 @@ class GridNeRFHIP:
             # ms; of 4096: 3.99 -> 3.77, the GPU is then the limit)
             full = N // step
             done = []
-            if full:
-                caps = self.capacities(step, S)
-                ws = []
-                for i, lane in enumerate(lanes[:full]):
-                    with torch.cuda.stream(lane):
-                        ws.append(self.workspace(step, S, i, caps))
-                n = len(ws)
-                L.check(
-                    self.lib.lm_render_chunks(
-                        C.byref(self._model_struct(S, white_bg, caps)), rays.data_ptr(), full * step, step, n,
-                        (C.c_void_p * n)(*[lane.cuda_stream for lane in lanes[:n]]), (C.c_void_p * n)(*[w.data_ptr() for w in ws]),
-                        (C.c_size_t * n)(*[w.numel() for w in ws]), rgb.data_ptr(), depth.data_ptr(), counters.data_ptr(),
-                    ),
-                    "lm_render_chunks",
-                )
-                if caps != (0, 0):
-                    done = [(slice(i * step, (i + 1) * step), counters[i], caps) for i in range(full)]
-            if full < len(starts):
-                sl = slice(full * step, N)
-                with torch.cuda.stream(lanes[full % len(lanes)]):
-                    caps = self.render_into(rays[sl], rgb[sl], depth[sl], white_bg=white_bg, N_samples=N_samples, slot=full % len(lanes),
-                                            counters=counters[full])
-                done.append((sl, counters[full], caps))
-            for s in side:
-                current.wait_stream(s)
+            try:
+                if full:
+                    caps = self.capacities(step, S)
+                    ws = []
+                    for i, lane in enumerate(lanes[:full]):
+                        with torch.cuda.stream(lane):
+                            ws.append(self.workspace(step, S, i, caps))
+                    n = len(ws)
+                    L.check(
+                        self.lib.lm_render_chunks(
+                            C.byref(self._model_struct(S, white_bg, caps)), rays.data_ptr(), full * step, step, n,
+                            (C.c_void_p * n)(*[lane.cuda_stream for lane in lanes[:n]]), (C.c_void_p * n)(*[w.data_ptr() for w in ws]),
+                            (C.c_size_t * n)(*[w.numel() for w in ws]), rgb.data_ptr(), depth.data_ptr(), counters.data_ptr(),
+                        ),
+                        "lm_render_chunks",
+                    )
+                    if caps != (0, 0):
+                        done = [(slice(i * step, (i + 1) * step), counters[i], caps) for i in range(full)]
+                if full < len(starts):
+                    sl = slice(full * step, N)
+                    with torch.cuda.stream(lanes[full % len(lanes)]):
+                        caps = self.render_into(rays[sl], rgb[sl], depth[sl], white_bg=white_bg, N_samples=N_samples, slot=full % len(lanes),
+                                                counters=counters[full])
+                    done.append((sl, counters[full], caps))
+            finally:  # (a failed launch leaves the chunks before it in flight)
+                for s in side:
+                    current.wait_stream(s)
             self.finish_chunks(done, rays, rgb, depth, white_bg=white_bg, N_samples=N_samples)
             self.counters.copy_(counters[len(starts) - 1])
             return len(starts)

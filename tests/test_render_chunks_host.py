@@ -1,5 +1,6 @@
 """What render_chunks owes its caller around the library call, replayed on the host with stand-ins for the streams and the
-library (no GPU): the library reads the current device for its launches, so the model's device is current during the call."""
+library (no GPU): the library reads the current device for its launches, so the model's device is current during the call; and the
+current stream is behind every side stream however the call ends, because the buffers go back to the allocator then."""
 import contextlib
 import types
 
@@ -78,3 +79,17 @@ def test_the_models_device_is_current_during_the_library_call(model):
     assert _render(model) == 4
     assert ("lm_render_chunks", 1) in model.log and ("render_into", 1) in model.log
     assert M.torch.current_device == 0
+
+
+@pytest.mark.parametrize("fails", ["library", "last chunk"])
+def test_side_streams_are_waited_for_when_a_launch_fails(model, fails):
+    if fails == "library":
+        model.lib.lm_render_chunks = lambda *a: -4
+    else:
+        def render_into(*a, **k):
+            raise L.LandmarkError("no room")
+        model.render_into = render_into
+    with pytest.raises(L.LandmarkError):
+        _render(model)
+    for i in range(2):
+        assert ("wait_stream", "current", f"side{i}") in model.log
