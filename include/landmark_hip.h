@@ -355,7 +355,8 @@ int lm_render_route(const lm_model *model, int64_t N);
 /* lm_render for N rays in chunks of `step`, chunk i on streams[i % n_streams] with that stream's workspace (each as lm_render
  * needs it for `step` rays) and counter block counters + i * LM_STAT_WORDS.  The caller has cleared the blocks at a point that
  * every stream is behind, and waits for the streams before it reads anything or, if the call fails, frees anything: the chunks
- * before the failing one may still be in flight.  One call for what would be thousands of them
+ * before the failing one may still be in flight.  lm_model.events: every chunk records them all, so that they hold the stages
+ * of the last one, with other chunks' work between on the GPU; for stage times of their own use lm_render.  One call for what would be thousands of them
  * per second: a chunk of a few thousand rays takes the GPU less time than a scripting language takes to launch it. */
 int lm_render_chunks(const lm_model *m, const float *rays, int64_t N, int64_t step, int32_t n_streams, void *const *streams,
                      void *const *workspaces, const size_t *workspace_bytes, float *rgb_map, float *depth_map, uint32_t *counters);
