@@ -766,8 +766,18 @@ int lm_launch_march(const lm_model *m, const float *rays, const uint64_t *bitmap
     // few rays: a wave per ray, one launch-wide round trip per 64-sample word instead of one per four samples
     if (n_rays <= LM_RAYS_LIMIT)
         return lm_launch_march_wave(m, rays, bitmap, p_first, word_mask, ray_list, bins, n_rays, w_valid, acc, depth, app_cnt, p_end, n_marched, st);
+    // Up to four rays per quad of two workgroups per CU: no third workgroup, where the registers would allow one (fp16 tables of
+    // 16 channels and fewer, 153 registers).  With few rays it adds none in flight at the end, when only long ones are left, and
+    // shares the CU with them.  Whole calls, two / three per CU (and the plain sum, two per CU), us: city block of 256 samples per
+    // ray and 4096^2 planes 13 000 rays 377 / 387 (382), 60 000 710 / 735 (712), 120 000 1115 / 1140 (1121), 250 000 2100 / 2115 (2109);
+    // three 256^2 planes 13 000 226 / 237 (229), 60 000 569 / 584 (577), 120 000 948 / 948 (962), 250 000 1799 / 1768 (1833), 1 000 000
+    // 6759 / 6471 (6912); nine planes 13 000 279 / 292 (292), 60 000 597 / 610 (620), 120 000 943 / 933 (957); block-stacked 13 000
+    // 199 / 211, 120 000 627 / 655.  With a density projection the wait for its weights wants the third from earlier on
+    // (60 000 rays of 886 samples 1602 / 1618, 120 000 3080 / 2908): always three there.
+    const unsigned two = (unsigned)lm_persistent_blocks(2);
+    const unsigned most = !m->density_basis && n_rays <= two * (unsigned)kTile * 4u ? two : ~0u;
 #define LM_MARCH_ONE(T_, ROLL_)                                                                                            \
-    hipLaunchKernelGGL((k_march<T_, 4, ROLL_>), dim3(resident_grid(reinterpret_cast<const void *>(&k_march<T_, 4, ROLL_>))), \
+    hipLaunchKernelGGL((k_march<T_, 4, ROLL_>), dim3(std::min(most, resident_grid(reinterpret_cast<const void *>(&k_march<T_, 4, ROLL_>)))), \
                        dim3(kBlock), 0, st, m->geom, ps, m->density_basis, rays, bitmap,   \
                        p_first, word_mask, ray_list, bins, n_rays, queue, m->act, m->density_shift, m->distance_scale,            \
                        m->weight_thres, lm_stop_value(*m), w_valid, acc, depth, app_cnt, p_end, n_marched)

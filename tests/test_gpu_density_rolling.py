@@ -48,3 +48,21 @@ def test_render_depth_equals_the_lookup_per_sample(gpu_lib, dn, ndims, res, opt,
     # at most K * 2^-24 * sum |products| (below 1 here), times distance scale and path into the opacity, times far into depth
     k = dn * ndims * len(res)
     assert (out["depth_map"] - w["depth_map"]).abs().max().item() <= 4.5 * k * 2.0 ** -24 * p.distance_scale * 4.0
+
+
+def test_render_does_not_depend_on_the_number_of_workgroups(gpu_lib):
+    """fp16 tables of 16 channels march with two workgroups per CU up to a number of rays and with three above it"""
+    from landmark_amd.model import GridNeRFHIP
+
+    p = scenes.make_params(seed=6, gridSize=(18, 14, 16), near_far=[0.5, 4.5], n_importance=64, ndims=3, density_shift=0.0)
+    for t in p.density_plane:
+        t.mul_(6.0)
+    m = GridNeRFHIP(O.to_fp16_features(p), device="cuda", mlp_precision="f16")
+    limit = 2 * torch.cuda.get_device_properties(0).multi_processor_count * 64 * 4
+    rays = scenes.pinhole_rays(400, 400, 380.0, scenes.sphere_pose(2.5, 9)).cuda()[: limit + 65]
+    assert rays.shape[0] == limit + 65
+    whole, _ = m(rays, chunk=limit + 65)
+    for chunk in (limit, limit // 2 + 33):
+        parts, _ = m(rays, chunk=chunk)
+        assert torch.equal(parts["rgb_map"], whole["rgb_map"]) and torch.equal(parts["depth_map"], whole["depth_map"])
+    assert (whole["rgb_map"] != 1.0).any()
