@@ -18,24 +18,7 @@
 
 namespace {
 
-// ---- explicit coordinates ----------------------------------------------------------------
-template <typename T, int CFIX>  // CFIX > 0: every plane has CFIX channels
-__global__ __launch_bounds__(kBlock) void k_density_xyz(PlaneSet ps, const float *__restrict__ den_w,
-                                                        const float *__restrict__ xyz, uint64_t M,
-                                                        float *__restrict__ out, const uint32_t *__restrict__ skip) {
-    if (skip && *skip) return;  // other kernels have taken the points
-    const unsigned qlane = threadIdx.x & 3u, slot = threadIdx.x >> 2;
-    const uint64_t n_tiles = (M + kTile - 1) / kTile;
-    for (uint64_t tile = lm_xcd_swizzle(blockIdx.x, gridDim.x); tile < n_tiles; tile += gridDim.x) {
-        const uint64_t p = tile * kTile + slot;
-        if (p >= M) continue;
-        float q[4] = {xyz[3 * p], xyz[3 * p + 1], xyz[3 * p + 2], 0.0f};
-        const float s = CFIX > 0 ? density_sum_fixed<T, (CFIX > 0 ? CFIX : 16)>(ps, q, qlane, den_w)
-                                 : density_sum<T>(ps, q, qlane, den_w);
-        if (qlane == 0) out[p] = s;
-    }
-}
-
+// ---- explicit coordinates (density: lm_gather.h) ------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_app_xyz(PlaneSet ps, int K, const float *__restrict__ xyz, uint64_t M,
                                                     float *__restrict__ out) {
@@ -523,16 +506,19 @@ int lm_check_planes(const lm_plane *planes, int32_t n, int *dtype_out, int *K_ou
     return LM_OK;
 }
 
-// skip: null, or device memory that is not zero where the call is to do nothing
-int lm_launch_density_xyz(const lm_plane *planes, int32_t n_planes, int dtype, const float *density_basis, const float *xyz, int64_t M, float *out,
-                          const uint32_t *skip, hipStream_t st) {
+extern "C" int lm_gather_density_xyz(const lm_plane *planes, int32_t n_planes, const float *density_basis,
+                                     const float *xyz, int64_t M, float *out, void *stream) {
+    int dtype;
+    if (int rc = lm_check_planes(planes, n_planes, &dtype, nullptr)) return rc;
+    LM_REQUIRE(M >= 0, "negative count");
+    if (M == 0) return LM_OK;
+    LM_REQUIRE(xyz && out, "null buffer");
     const PlaneSet ps = make_set(planes, n_planes);
-    const uint64_t tiles = ((uint64_t)M + kTile - 1) / kTile;
-    const unsigned grid = (unsigned)std::min<uint64_t>(tiles, (uint64_t)lm_persistent_blocks(8));
-    bool all64 = true;
-    for (int k = 0; k < n_planes; ++k) all64 &= planes[k].C == 64;
-#define LM_DX(T_, C_) \
-    hipLaunchKernelGGL((k_density_xyz<T_, C_>), dim3(grid), dim3(kBlock), 0, st, ps, density_basis, xyz, (uint64_t)M, out, skip)
+    const unsigned grid = density_xyz_grid(M);
+    const bool all64 = planes_all_64(planes, n_planes);
+#define LM_DX(T_, C_)                                                                                                    \
+    hipLaunchKernelGGL((k_density_xyz<T_, C_, false>), dim3(grid), dim3(kBlock), 0, (hipStream_t)stream, ps, density_basis, xyz, \
+                       (uint64_t)M, out, nullptr)
     if (dtype == LM_F32) {
         if (all64) LM_DX(float, 64); else LM_DX(float, 0);
     } else {
@@ -541,16 +527,6 @@ int lm_launch_density_xyz(const lm_plane *planes, int32_t n_planes, int dtype, c
 #undef LM_DX
     LM_CHECK_LAUNCH("k_density_xyz");
     return LM_OK;
-}
-
-extern "C" int lm_gather_density_xyz(const lm_plane *planes, int32_t n_planes, const float *density_basis,
-                                     const float *xyz, int64_t M, float *out, void *stream) {
-    int dtype;
-    if (int rc = lm_check_planes(planes, n_planes, &dtype, nullptr)) return rc;
-    LM_REQUIRE(M >= 0, "negative count");
-    if (M == 0) return LM_OK;
-    LM_REQUIRE(xyz && out, "null buffer");
-    return lm_launch_density_xyz(planes, n_planes, dtype, density_basis, xyz, M, out, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int lm_gather_app_xyz(const lm_plane *planes, int32_t n_planes, const float *xyz, int64_t M, float *out,

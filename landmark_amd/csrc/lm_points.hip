@@ -598,8 +598,6 @@ bool plan_density(const lm_plane *planes, int n, int64_t M, Plan &pn) {
 }  // namespace
 
 int lm_check_planes(const lm_plane *planes, int32_t n, int *dtype_out, int *K_out);
-int lm_launch_density_xyz(const lm_plane *planes, int32_t n_planes, int dtype, const float *density_basis, const float *xyz, int64_t M, float *out,
-                          const uint32_t *skip, hipStream_t st);
 
 // Where it pays.  Whole calls with k_density_xyz / here, three planes, evenly spread points in no order: 2048^2 x 64 channels,
 // 2^24 points 8800 / 3200 us, 6 million 3310 / 1740, 3 million (fewer than texels) 1690 / 1560; 1000^2 x 32, 2^24 points 4870 /
@@ -648,12 +646,16 @@ extern "C" int lm_gather_density_binned(const lm_plane *planes, int32_t n_planes
     const size_t order_step = (size_t)pn.slice, tab_step = (size_t)pn.max_units * (pn.max_subs + 1);
     const PlaneSet ps = make_set(planes, n_planes);
     const unsigned grid = (unsigned)(lm_persistent_blocks(3) / LM_XCDS * LM_XCDS);  // as many as LDS lets live at once
+    const bool all64 = planes_all_64(planes, n_planes);
+#define LM_DX(C_)                                                                                                            \
+    hipLaunchKernelGGL((k_density_xyz<float, C_, true>), dim3(density_xyz_grid(m)), dim3(kBlock), 0, st, ps, density_basis, pts, \
+                       (uint64_t)m, out + at, flag)
     for (int64_t at = 0; at < M; at += pn.slice) {
         const uint32_t m = (uint32_t)std::min(pn.slice, M - at);
         const float *pts = xyz + 3 * at;
         const unsigned wgs = (m + kUnit - 1) / kUnit;
         hipLaunchKernelGGL(k_bin_decide, dim3(1), dim3(kScatter), 0, st, pn.axes, pts, m, counts, bins, queue, flag);
-        if (int rc = lm_launch_density_xyz(planes, n_planes, dtype, density_basis, pts, m, out + at, flag, st)) return rc;
+        if (all64) LM_DX(64); else LM_DX(0);
         hipLaunchKernelGGL(k_bin_count, dim3(std::min(wgs, (unsigned)lm_persistent_blocks(1))), dim3(kScatter), 0, st, flag, side, pts, m, counts);
         hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kScatter), 0, st, flag, side, pn.axes, counts, units, n_units, groups, pn.max_groups, n_groups);
         hipLaunchKernelGGL(k_bin_scatter, dim3(wgs), dim3(kScatter), 0, st, flag, side, pts, m, counts, rec);
@@ -679,6 +681,7 @@ extern "C" int lm_gather_density_binned(const lm_plane *planes, int32_t n_planes
             col += p.C;
         }
     }
+#undef LM_DX
     LM_CHECK_LAUNCH("k_bin_density");
     return LM_OK;
 }
