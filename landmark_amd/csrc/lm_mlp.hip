@@ -265,18 +265,18 @@ __device__ __forceinline__ void colour_layers(const typename Mma<PREC>::frag *w1
 #pragma unroll
             for (int k = 0; k < 3; ++k) out[cb][k] = colour_of<PREC>(last_layer_sum(part[0][k], part[1][k], part[2][k], part[3][k], b3[k]));
         }
-        return;
+    } else {
+        floatx16 acc3[1][NCB];
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) acc3[0][cb] = load_bias(b3, h);
+        dense_layer<PREC, 1, NCB, T2, 4>(w3, 0, lane, b3frag, acc3);
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                out[cb][k] = colour_of<PREC>(acc3[0][cb][k]);
+            }
     }
-    floatx16 acc3[1][NCB];
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) acc3[0][cb] = load_bias(b3, h);
-    dense_layer<PREC, 1, NCB, T2, 4>(w3, 0, lane, b3frag, acc3);
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            out[cb][k] = colour_of<PREC>(acc3[0][cb][k]);
-        }
 }
 
 // The three layers of the 16-bit and split modes as one stream of matrix steps.  A "job" is one block of 32 output
