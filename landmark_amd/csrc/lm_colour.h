@@ -187,8 +187,9 @@ __device__ __forceinline__ void encode_inputs(const float (*raw)[16],
 
 // fp32 mode: a 32-row block of the last layer's input (the lane's 16 values after relu) times its three rows of weights, for the
 // vector unit: `w` gives {row 0, row 1, row 2, -} of slot v.  A matrix instruction would work 32 rows for these three (64 of them
-// a tile, a tenth of the network's): with the steps of the all-zero input slots left out too, 2^22 rows 2633 -> 2464 us; 1024
-// rays, where one wave did these steps alone, 48.4 -> 45.5 (whole call).  The blocks' sums are added in order, then the halves', then the bias (last_layer_sum), in every kernel.
+// a tile, a tenth of the network's).  2^22 rows 2616 -> 2439 us, and 2355 with the steps of the all-zero input slots left out;
+// 1024 rays, where one wave did these steps alone, 49.9 -> 44.6 and 44.2 (whole call, with the rays kernel's 32-bit offsets).
+// The blocks' sums are added in order, then the halves', then the bias (last_layer_sum), in every kernel.
 template <typename W> __device__ __forceinline__ void last_layer_block(const float *x, const W &w, float *sum) {
     sum[0] = sum[1] = sum[2] = 0.0f;
 #pragma unroll

@@ -349,11 +349,12 @@ __device__ __forceinline__ void density_sum_n(const PlaneSet &ps, const float *q
 
 // density_sum_n of four samples for planes of one channel group per lane and tables below 4 GB (density_rolls): the next plane's
 // footprints are worked out while this one's loads travel, and its loads are issued as soon as products have left the
-// registers (all four samples' in fp32, two at a time in fp16).  Offsets are 32-bit bytes from the plane's (scalar) address:
+// registers (all four samples' at once with 16-byte loads, two at a time with 8-byte ones).  Offsets are 32-bit bytes from the plane's (scalar) address:
 // a seventh of the march's vector instructions less (3.54 -> 3.03 G on the frame below, its loads 170 -> 152 M) and 202 instead of
 // 231 registers.  Same operations per sample, hence the same bits.
-// 960 x 540 rays of 3544 samples, three fp32 planes with a projection: frame 26.1 -> 22.5 ms (march 13.2 -> 10.1); 4K city (fp16)
-// 39.7 -> 39.0 ms; frames bound by bytes 1 %.  Two samples at a time in fp32 too 23.0, one
+// 960 x 540 rays of 3544 samples, three fp32 planes with a projection, one view: frame 26.1 -> 22.5 ms (march 13.2 -> 10.1; over the
+// views of an orbit 29.5 -> 25.3); 4K city (fp16) 39.7 -> 39.0 ms; frames bound by bytes the same within 0.5 %
+// (a tenth more lines fetched, at a higher rate).  Two samples at a time in fp32 too 23.0, one
 // 23.5; the same without work on the next plane 24.5.  The projection's weights are loaded once per plane: once per sample is
 // what the compiler made of the plain form, and that took 30.0.
 struct RollTaps {

@@ -15,10 +15,10 @@
 // XCD at about the same time and stay in its L2, so that records are read from memory once per plane whatever the order
 // within a unit.  A block of too many points becomes several units, a column of many units several groups, and a sub-tile
 // with few points is not staged, its points read the table directly.
-// 2^24 points, three planes of 2048^2 x 64 channels: 8.8 -> 3.2 ms (sorting 0.65, planes 0.81 + 0.85 + 1.12; the last writes
-// 4 bytes per point anywhere in 64 MB).  What bounds a plane: 2 KB of LDS reads and 512 bytes of line texels per point, 45
+// 2^24 points, three planes of 2048^2 x 64 channels: 8.8 -> 3.2 ms (kernel trace: sorting 0.58, planes 0.77 + 0.84 + 1.12; the last
+// writes 4 bytes per point anywhere in 64 MB).  What bounds a plane: 2 KB of LDS reads and 512 bytes of line texels per point, 45
 // vector instructions per four points, each 0.25 - 0.4 ms by itself, and the round trip task -> units -> order -> record -> line
-// of a workgroup that lives 15 us, three to a compute unit.  Measured on the way: records sorted again per orientation instead
+// of a task that takes 15 us, three workgroups to a compute unit.  Measured on the way: records sorted again per orientation instead
 // of 16-bit positions 3.6 ms (moving 20 bytes per point cost more than the planes' locality gained); texels through registers
 // in a loop over tasks 3.8 (spills); two texel halves per lane (8 lanes per point) 3.7; line texels two points ahead 3.3.
 #include <algorithm>
@@ -66,8 +66,9 @@ struct Axes {
 };
 
 // One workgroup looks at kSample points and their successors: *flag = 1 if fewer than one in eight shares its 1 / 64 x 1 / 64 of
-// the first plane with its successor, and no such part of a plane holds more than kCrowd points of the sample (one on average;
-// points spread evenly do not reach ten).  It also clears the counters.
+// the first plane with its successor, and no such part of a plane holds more than kCrowd points of the sample (one on average:
+// of 4096 evenly spread points some part on one of three orientations gets more than 16 once in 7e10 calls, ten or more once in
+// 700).  It also clears the counters.
 constexpr int kSample = 4096, kCells = 64, kCrowd = 16;
 __global__ __launch_bounds__(kScatter) void k_bin_decide(Axes axes, const float *__restrict__ xyz, uint32_t M, uint32_t *__restrict__ counts,
                                                          int n_counts, uint32_t *__restrict__ queue, uint32_t *__restrict__ flag) {
@@ -602,9 +603,9 @@ int lm_check_planes(const lm_plane *planes, int32_t n, int *dtype_out, int *K_ou
 // Where it pays.  Whole calls with k_density_xyz / here, three planes, evenly spread points in no order: 2048^2 x 64 channels,
 // 2^24 points 8800 / 3200 us, 6 million 3310 / 1740, 3 million (fewer than texels) 1690 / 1560; 1000^2 x 32, 2^24 points 4870 /
 // 2240; 512^2 x 64, 2^24 points 6940 / 2710.  Points that k_bin_decide sends back cost 40 - 60 us more than without a look:
-// 2^24 points in a twentieth of the box 4037 / 4077, all at one place 2146 / 2207, on a lattice in its order 4244 / 4290.  That
-// is to stay in the noise of a call, so the line lies at 1.2e9 channels (6 million points of 192), where calls take 0.8 - 3.3
-// ms; below it the gain would reach further down (2 million points of 512^2 x 64 860 / 430).
+// 2^24 points in a twentieth of the box 4037 / 4077, all at one place 2146 / 2207, on a lattice in its order 4244 / 4290.  The line
+// at 1.2e9 channels (6 million points of 192) keeps that to a fifteenth of the shortest call that gains nothing (0.8 ms; others take
+// up to 3.3 ms); below it evenly spread points would still gain (2 million points of 512^2 x 64 860 / 430).
 static bool density_pays(const lm_plane *planes, int n, int64_t M) {
     int64_t channels = 0, bytes = 0, texels = 0;
     for (int k = 0; k < n; ++k) {
